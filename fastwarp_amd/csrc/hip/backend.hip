@@ -352,20 +352,10 @@ HImage HipBackend::upload_image(const Image& v) {
   HostTimer host_timer("upload_image");
   const size_t n = v.grid.num_voxels();
   auto* stage = static_cast<float*>(ctx_->pinned(n * sizeof(float)));
-  constexpr size_t kGrain = size_t(1) << 16;
-  std::vector<float> bound((n + kGrain - 1) / kGrain, 0.0f);
-  parallel_chunks(n, kGrain, [&](size_t c, size_t b, size_t e) {
-    float m = 0.0f;
-    for (size_t i = b; i < e; ++i) {
-      const float x = float(v.data[i]);
-      stage[i] = x;
-      if (std::isfinite(x)) m = std::max(m, std::fabs(x));
-    }
-    bound[c] = m;
+  parallel_for(n, [&](size_t b, size_t e) {
+    for (size_t i = b; i < e; ++i) stage[i] = float(v.data[i]);
   });
-  float m = 0.0f;
-  for (float x : bound) m = std::max(m, x);
-  HImage im{v.grid, DevBuf(ctx_.get(), n), m};
+  HImage im{v.grid, DevBuf(ctx_.get(), n)};
   check(hipMemcpyAsync(im.buf.get(), stage, n * sizeof(float), hipMemcpyHostToDevice, ctx_->stream()), "upload image");
   ctx_->sync();
   return im;
@@ -376,7 +366,7 @@ HImage HipBackend::resample_isotropic(const HImage& im, double mm) {
   const Grid& g = im.grid;
   const size_t n = g.num_voxels();
   if (std::fabs(g.spacing[0] - mm) < 1e-6 && std::fabs(g.spacing[1] - mm) < 1e-6 && std::fabs(g.spacing[2] - mm) < 1e-6) {
-    HImage copy{g, DevBuf(ctx_.get(), n), im.bound};
+    HImage copy{g, DevBuf(ctx_.get(), n)};
     check(hipMemcpyAsync(copy.buf.get(), im.buf.get(), n * sizeof(float), hipMemcpyDeviceToDevice, ctx_->stream()), "copy image");
     return copy;
   }
@@ -400,7 +390,7 @@ HImage HipBackend::resample_isotropic(const HImage& im, double mm) {
   check(hipMemcpyAsync(tables.get(), lo.data(), lo.size() * sizeof(int), hipMemcpyHostToDevice, ctx_->stream()), "upload table");
   check(hipMemcpyAsync(tables.get() + lo.size(), fr.data(), fr.size() * sizeof(float), hipMemcpyHostToDevice, ctx_->stream()),
         "upload table");
-  HImage r{og, DevBuf(ctx_.get(), og.num_voxels()), im.bound};
+  HImage r{og, DevBuf(ctx_.get(), og.num_voxels())};
   {
     // the source read once (at most), the result written
     Timed t(*ctx_, "k_resample_iso", 4.0 * double(og.num_voxels()) + 4.0 * std::min(double(n), double(og.num_voxels())));
@@ -414,17 +404,7 @@ HImage HipBackend::resample_isotropic(const HImage& im, double mm) {
 
 HImage HipBackend::upload_image_f32(const Grid& g, const float* data) {
   const size_t n = g.num_voxels();
-  constexpr size_t kGrain = size_t(1) << 16;
-  std::vector<float> bound((n + kGrain - 1) / kGrain, 0.0f);
-  parallel_chunks(n, kGrain, [&](size_t c, size_t b, size_t e) {
-    float m = 0.0f;
-    for (size_t i = b; i < e; ++i)
-      if (std::isfinite(data[i])) m = std::max(m, std::fabs(data[i]));
-    bound[c] = m;
-  });
-  float m = 0.0f;
-  for (float x : bound) m = std::max(m, x);
-  HImage im{g, DevBuf(ctx_.get(), n), m};
+  HImage im{g, DevBuf(ctx_.get(), n)};
   check(hipMemcpyAsync(im.buf.get(), data, n * sizeof(float), hipMemcpyHostToDevice, ctx_->stream()), "upload image");
   ctx_->sync();
   return im;
@@ -524,7 +504,7 @@ WarpArgs warp_args(const Grid& src, const HField& field, const HField* pre, cons
 
 HImage HipBackend::warp_through_field(const HImage& src, const HField& field, const HField* pre, const AffineTransform* affine) {
   WarpArgs a = warp_args(src.grid, field, pre, affine);
-  HImage out{field.grid, DevBuf(ctx_.get(), field.grid.num_voxels()), src.bound};
+  HImage out{field.grid, DevBuf(ctx_.get(), field.grid.num_voxels())};
   a.src = src.buf.get();
   a.out = out.buf.get();
   const double no = double(field.grid.num_voxels());
@@ -539,7 +519,7 @@ std::pair<HImage, HImage> HipBackend::warp_pair(const HImage& src0, const HField
     return {warp_through_field(src0, field0, nullptr, affine0), warp_through_field(src1, field1, nullptr, affine1)};
   WarpArgs a0 = warp_args(src0.grid, field0, nullptr, affine0), a1 = warp_args(src1.grid, field1, nullptr, affine1);
   const Grid& g = field0.grid;
-  HImage out0{g, DevBuf(ctx_.get(), g.num_voxels()), src0.bound}, out1{g, DevBuf(ctx_.get(), g.num_voxels()), src1.bound};
+  HImage out0{g, DevBuf(ctx_.get(), g.num_voxels())}, out1{g, DevBuf(ctx_.get(), g.num_voxels())};
   a0.src = src0.buf.get();
   a0.out = out0.buf.get();
   a1.src = src1.buf.get();
@@ -558,14 +538,13 @@ HImage HipBackend::warp_mask_through_field(const HImage& mask, const HField& fie
   a.nearest = 1;
   if (product) {
     HImage out = std::move(*product);
-    out.bound *= mask.bound;
     a.product = out.buf.get();
     a.out = out.buf.get();
     Timed t(*ctx_, "k_warp", 24.0 * double(field.grid.num_voxels()));
     launch_warp(a, ctx_->stream());
     return out;
   }
-  HImage out{field.grid, DevBuf(ctx_.get(), field.grid.num_voxels()), mask.bound};
+  HImage out{field.grid, DevBuf(ctx_.get(), field.grid.num_voxels())};
   a.out = out.buf.get();
   Timed t(*ctx_, "k_warp", 20.0 * double(field.grid.num_voxels()));
   launch_warp(a, ctx_->stream());
@@ -591,12 +570,7 @@ MetricPair<HField> HipBackend::cc_pair(const HImage& fixed, const HImage& moving
   a.valid = valid ? valid->buf.get() : nullptr;
   a.d = dims_of(g);
   a.radius = int(radius);
-  a.tile_z = cc_tile_for(a.d, int(ctx_->tuning().get("cc.tile_z", n, cc_tile_z)),
-                         int(ctx_->tuning().get("cc.min_blocks", n, 512)));
-  a.scale_f = cc_split_scale(fixed.bound);
-  a.scale_m = cc_split_scale(moving.bound);
-  a.step_f = 1.0f / a.scale_f;
-  a.step_m = 1.0f / a.scale_m;
+  a.tile_z = cc_tile(ctx_->tuning(), a.d, a.radius);
   a.probes = probes_of(g);
   a.d_fixed = out.fields[0].buf.get();
   a.d_moving = out.fields[1].buf.get();
@@ -671,12 +645,7 @@ MetricPair<HField> HipBackend::cc_pair_deferred(const HImage& fixed, const HImag
   a.valid = nullptr;
   a.d = dims_of(g);
   a.radius = int(radius);
-  a.tile_z = cc_tile_for(a.d, int(ctx_->tuning().get("cc.tile_z", n, cc_tile_z)),
-                         int(ctx_->tuning().get("cc.min_blocks", n, 512)));
-  a.scale_f = cc_split_scale(fixed.bound);
-  a.scale_m = cc_split_scale(moving.bound);
-  a.step_f = 1.0f / a.scale_f;
-  a.step_m = 1.0f / a.scale_m;
+  a.tile_z = cc_tile(ctx_->tuning(), a.d, a.radius);
   a.probes = probes_of(g);
   a.d_fixed = out.fields[0].buf.get();
   a.d_moving = out.fields[1].buf.get();
@@ -771,7 +740,7 @@ HImage HipBackend::smooth_image(const HImage& src, double sigma, SigmaUnits unit
 HImage HipBackend::smooth_image_mm(const HImage& src, const Vec3& sigma_mm) {
   const Grid& g = src.grid;
   const size_t n = g.num_voxels();
-  HImage out{g, DevBuf(ctx_.get(), n), src.bound};
+  HImage out{g, DevBuf(ctx_.get(), n)};
   hipStream_t s = ctx_->stream();
   if (!(sigma_mm[0] > 0.0 || sigma_mm[1] > 0.0 || sigma_mm[2] > 0.0)) {
     check(hipMemcpyAsync(out.buf.get(), src.buf.get(), n * sizeof(float), hipMemcpyDeviceToDevice, s), "copy image");
@@ -893,7 +862,7 @@ HImage HipBackend::preprocess_image(const HImage& raw, float lower, float upper,
   const IntensityWindow w = intensity_window(h, lower, upper, out_min, out_max);
   const float sh = float(w.scale), th_ = float(w.shift);
   const float sl = float(w.scale - double(sh)), tl = float(w.shift - double(th_));
-  HImage out{g, DevBuf(ctx_.get(), size_t(n)), float(std::max(std::fabs(out_min), std::fabs(out_max)))};
+  HImage out{g, DevBuf(ctx_.get(), size_t(n))};
   {
     Timed t(*ctx_, "k_window", 8.0 * double(n));
     launch_window(raw.buf.get(), out.buf.get(), n, float(w.lo), float(w.hi), sh, sl, th_, tl, float(out_min), float(out_max), s);

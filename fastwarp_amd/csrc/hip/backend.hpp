@@ -9,6 +9,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 #include <map>
 #include <memory>
@@ -221,13 +222,22 @@ class DevBuf {
 // tuning/gfx950.json beside the library's directory (fastwarp_amd/tuning/ for lib/), else empty.
 const TuningTable& default_tuning();
 
-// A scalar image on the device (f32, x-fastest) with an upper bound of |value| (taken on the host
-// at upload and carried through the ops that cannot grow it: warps, smoothing, resampling). The
-// CC sums split every value at a power-of-two step of this bound.
+// The planes a CC block walks on grid d under tuning table t (knobs cc.tile_z, cc.min_blocks; the
+// split that takes the least time where neither is set).
+// The kernel addresses a tile's rows with 32-bit byte offsets from the first.
+inline int cc_tile(const TuningTable& t, const Dims& d, int radius) {
+  if (4ll * d.nx * std::min(kCcTileY + 2 * radius, d.ny) >= (1ll << 32))
+    invalid("hip backend", "cc: rows of " + std::to_string(d.nx) + " voxels are not supported");
+  const uint64_t n = uint64_t(d.n());
+  const int tile = int(t.get("cc.tile_z", n, 0)), blocks = int(t.get("cc.min_blocks", n, 0));
+  if (tile == 0 && blocks == 0) return cc_tile_for(d, radius, 0, 0);
+  return cc_tile_for(d, radius, tile ? tile : kCcTileZ, blocks ? blocks : kCcMinBlocks);
+}
+
+// A scalar image on the device (f32, x-fastest).
 struct HImage {
   Grid grid;
   DevBuf buf;
-  float bound = 0.0f;
 };
 
 // A displacement field on the device: three f32 planes x, y, z.
@@ -285,7 +295,7 @@ class HipBackend {
                              size_t bins, bool want_norms);
 
   // Level smoothing on the device (pyramid.rs:429-465, f32 recursive Gaussian, axes z, x, y);
-  // sigma <= 0 gives a copy. The result's bound is its measured maximum magnitude.
+  // sigma <= 0 gives a copy.
   HImage smooth_image(const HImage& src, double sigma, SigmaUnits units);
   HImage smooth_image_mm(const HImage& src, const Vec3& sigma_mm);
   // Nearest-voxel and linear values at physical points (NaN outside), as the linear stages'
@@ -336,8 +346,6 @@ class HipBackend {
   void settle() { ctx_->settle(); }
   HField resample_field(const HField& field, const Grid& grid);
 
-  // CC tile height in z of the fused kernel.
-  int cc_tile_z = kCcTileZ;
   // Slots of the coherent-host rings of update maxima and CC partials (results awaiting a settle).
   static constexpr size_t kMaximaSlots = 64;
   static constexpr size_t kCcSlots = 4;

@@ -226,8 +226,8 @@ std::unique_ptr<LevelBuffers> make_level_buffers(HipBackend& b, const SynRecipe&
   L->dmov.resize(k);
   for (size_t q = 0; q < k; ++q)
     for (size_t c = 0; c < nc; ++c) {
-      L->fmid[q].push_back(HImage{g, DevBuf(&ctx, n), 0.0f});
-      L->mmid[q].push_back(HImage{g, DevBuf(&ctx, n), 0.0f});
+      L->fmid[q].push_back(HImage{g, DevBuf(&ctx, n)});
+      L->mmid[q].push_back(HImage{g, DevBuf(&ctx, n)});
       L->dfix[q].push_back(HField{g, DevBuf(&ctx, 3 * n)});
       L->dmov[q].push_back(HField{g, DevBuf(&ctx, 3 * n)});
     }
@@ -245,7 +245,7 @@ std::unique_ptr<LevelBuffers> make_level_buffers(HipBackend& b, const SynRecipe&
   }
   L->step_parts = DevBuf(&ctx, k * 4 * size_t(L->nb));
   L->factors = DevBuf(&ctx, 2 * k);
-  L->tile_z = cc_tile_for(d, int(ctx.tuning().get("cc.tile_z", n, b.cc_tile_z)), int(ctx.tuning().get("cc.min_blocks", n, 512)));
+  L->tile_z = cc_tile(ctx.tuning(), d, int(recipe.cc_radius));
   const dim3 gr = cc_grid(d, L->tile_z);
   L->blocks = size_t(gr.x) * gr.y * gr.z;
   // coherent host memory for the whole level (later, smaller active sets fit in it)
@@ -345,8 +345,6 @@ void issue_updates(HipBackend& b, const SynRecipe& recipe, const std::vector<dou
       const Subject& u = subj[act[q]];
       const HImage& F = *smooth[act[q]][c].fixed;
       const HImage& M = *smooth[act[q]][c].moving;
-      L.fmid[q][c].bound = F.bound;
-      L.mmid[q][c].bound = M.bound;
       wf.a[q] = warp_args(F.grid, *u.f2m_inv, nullptr, nullptr);
       wf.a[q].src = F.buf.get();
       wf.a[q].out = L.fmid[q][c].buf.get();
@@ -372,11 +370,6 @@ void issue_updates(HipBackend& b, const SynRecipe& recipe, const std::vector<dou
       a.d = d;
       a.radius = int(recipe.cc_radius);
       a.tile_z = L.tile_z;
-      a.scale_f = cc_split_scale(L.fmid[q][c].bound);
-      a.scale_m = cc_split_scale(L.mmid[q][c].bound);
-      a.step_f = 1.0f / a.scale_f;
-      a.step_m = 1.0f / a.scale_m;
-      a.bounds = nullptr;
       a.probes = probes_of(g);
       a.d_fixed = L.dfix[q][c].buf.get();
       a.d_moving = L.dmov[q][c].buf.get();

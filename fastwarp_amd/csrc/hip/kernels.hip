@@ -11,6 +11,7 @@
 
 #include <cfloat>
 #include <climits>
+#include <type_traits>
 
 #include "device_common.hpp"
 #include "fastdiv.hpp"
@@ -25,61 +26,160 @@ LaunchEvents*& current_launch_events() {
 // ------------------------------------------------------------------------------------------
 // CC pair (metric/cc.rs:170-321 and wgpu_backend.rs:1354-1520 semantics, fused).
 //
-// The window sums are those of the f32 voxel values with f64 precision and no rounding history:
-// each value is split at a power-of-two step of its image's bound (v = h q + l, h an integer), the
-// integer parts are summed exactly in f64 and the remainders in f64 beside them, and the two are
-// combined once per window. So a window of zeros sums to zero (as the oracle's direct box sums do,
-// which matters for its degenerate-window rule), and a window of tiny values (the edge of a
-// zero-padded region, where the local variance is 1e-12 and the coefficient is the largest of the
-// image) keeps its relative precision, which a fixed-point quantisation at the bound loses. On
-// gfx950 the vector FP64 rate equals the non-packed FP32 rate. The centred moments, the local CC
-// and the coefficients follow cc.rs:270-300 in f64; the derivative is the coefficient times the
-// f32 central difference, rounded once to f32. Each output voxel writes both derivative
-// directions; localCC is symmetric, so one value partial serves both.
+// The window sums of a, b, aa, bb and ab are taken in f64, every window from its own terms: the
+// product of two f32 values is exact in f64, and no sum is ever formed by subtracting a plane that
+// has left the window. So a window of zeros sums to exactly zero (which decides the degenerate
+// windows of cc.rs:270-300), a window of tiny values (the smoothed edge of a zero-padded region,
+// local variance 1e-12, where the coefficient is the largest of the image) keeps its relative
+// precision, and no scale of the image enters. The centred moments, the local CC and the
+// coefficients follow in f64 from one reciprocal; the derivative is the coefficient times the f32
+// central difference, rounded once to f32. Each output voxel writes both derivative directions;
+// localCC is symmetric, so one value partial serves both.
 //
-// A block owns a 64 x 8 (x, y) tile over a run of tile_z planes. Each thread keeps the running
-// z-window sums of its columns of the tile and halo in registers: one plane enters and one leaves
-// per step, read from global memory (the leaving plane was read 2r+1 steps before and sits in
-// cache). The z sums of the step's plane go to LDS; the x pass sums pairs of outputs along x
-// (sharing their middle 2r columns, summed directly) and writes its sums back over the z sums after
-// a barrier, so one LDS buffer serves both passes; the y pass sums 2r+1 rows per output voxel.
+// A block owns a 32 x 8 (x, y) tile over a run of tile_z planes and takes the planes z0 - R ..
+// z1 - 1 + R in turn. A plane's tile and halo are staged in LDS as f32 (the next plane's loads are in
+// flight meanwhile); the x pass forms the products and sums them over x, eight outputs a lane, whose
+// windows share their middle (2.6 additions an output where the plain sum takes 8), a wave for each
+// of (a, aa), (b, bb), (ab); the y pass adds 2R + 1 rows of x sums per output voxel; the z pass
+// keeps the last planes' x/y sums of the thread's one output column in registers and forms the
+// running window from partial sums (three or four additions a plane, CcWindow).
+//
+// Bound by the latency of its f64 chains at two waves a SIMD (vector instructions fill a third of the
+// time, the LDS reads of the y pass another). 182 x 218 x 182, radius 4, with the value's sum: 156 us;
+// sums of split values, running along z with the leaving plane subtracted, on 64 x 8 tiles: 375 us
+// (radius 2: 120 for 305, radius 8: 329 for 952; 45 x 54 x 45 at radius 4: 22 for 51).
 // ------------------------------------------------------------------------------------------
-constexpr int kCcTX = 64, kCcTY = 8;
+constexpr int kCcTX = 32, kCcTY = kCcTileY, kCcThreads = kCcTX * kCcTY;
+constexpr int kCcRun = 8;  // outputs along x of one lane of the x pass
 
-// Threads per block: one per output voxel of the 64 x 8 tile. Each thread owns up to
-// ceil((64 + 2R) (8 + 2R) / 512) tile-and-halo columns (three at radius 4); the running sums of a
-// column take 20 registers, which leaves one block of eight waves per CU.
 template <int R>
-constexpr int cc_threads() {
-  return kCcTX * kCcTY;
+struct CcTile {
+  static constexpr int W = 2 * R + 1;
+  static constexpr int LX = kCcTX + 2 * R, LY = kCcTY + 2 * R;
+  // a row is read in 16-byte vectors; an odd number of them a row keeps neighbouring rows' reads
+  // on different banks
+  static constexpr int VEC = (LX + 3) / 4;
+  static constexpr int PITCH = 4 * (VEC % 2 ? VEC : VEC + 1);
+  static constexpr int PER = (LX * LY + kCcThreads - 1) / kCcThreads;  // elements a thread stages
+  static constexpr int RUNS = kCcTX / kCcRun, JOBS = RUNS * LY;
+  // Column tx of row ly of the x sums is stored in another 16-byte place of its 64 bytes: the lanes
+  // of the x pass store 64 bytes apart, and the exchange spreads eight of them (four runs of two
+  // rows) over all banks. A row stays the same 256 bytes, so the y pass reads it without conflicts.
+  static __device__ __forceinline__ int swap_of(int ly, int run) { return (run >> 1) | ((ly & 1) << 1); }
+  static __device__ __forceinline__ int column(int ly, int tx) {
+    return tx ^ (swap_of(ly, tx / kCcRun) << 1);
+  }
+  // the f32 inputs of a run of outputs
+  static constexpr int N = kCcRun + 2 * R;
+  static __device__ __forceinline__ void read_run(const float* p, float (&f)[(N + 3) / 4 * 4]) {
+#pragma unroll
+    for (int q = 0; q < (N + 3) / 4; ++q) *reinterpret_cast<float4*>(f + 4 * q) = *reinterpret_cast<const float4*>(p + 4 * q);
+  }
+  static __device__ __forceinline__ void write_run(double* row, int ly, int run, const double (&o)[kCcRun]) {
+    const int s = swap_of(ly, run);
+#pragma unroll
+    for (int p = 0; p < kCcRun / 2; ++p)
+      *reinterpret_cast<double2*>(row + run * kCcRun + 2 * (p ^ s)) = make_double2(o[2 * p], o[2 * p + 1]);
+  }
+};
+
+// o[i] = sum of the terms i .. i + W - 1: groups of at most W outputs share the middle of their
+// windows and add running sums of the ends to it. add(t, s) gives s plus term t (a product goes
+// into the sum by one fma, so it is not rounded by itself), first(t) the term alone.
+template <int N, int W, typename V, typename First, typename Add>
+__device__ __forceinline__ void window_sums(First first, Add add, V (&o)[N]) {
+#pragma unroll
+  for (int base = 0; base < N; base += W) {
+    const int n = N - base < W ? N - base : W;
+    V left = first(base + n - 1);
+#pragma unroll
+    for (int t = n; t < W; ++t) left = add(base + t, left);
+    o[base + n - 1] = left;
+#pragma unroll
+    for (int i = n - 2; i >= 0; --i) {
+      left = add(base + i, left);
+      o[base + i] = left;
+    }
+    V right = V(0);
+#pragma unroll
+    for (int i = 1; i < n; ++i) {
+      right = i == 1 ? first(base + W) : add(base + W - 1 + i, right);
+      o[base + i] += right;
+    }
+  }
 }
 
-// Central differences along the three physical axes on an axis-aligned grid (probes at +-0.5 on
-// one grid axis each): the difference of the two linear interpolations is half the difference of
-// the two neighbours (the centre cancels), computed as such so that it carries one rounding.
-__device__ __forceinline__ void axis_gradient(const float* __restrict__ img, const Dims& d, const Probes& pr, int i, int j,
-                                              int k, float out[3]) {
-  const long long sy = d.nx, sz = (long long)d.nx * d.ny;
-  const float* p = img + lin(d, i, j, k);
-  const int pos[3] = {i, j, k};
-  const int len[3] = {d.nx, d.ny, d.nz};
-  const long long stride[3] = {1, sy, sz};
-  float half_diff[3];
+// The running window of the z pass over W planes of one sum: step<J>(w), J the plane's place in a cycle
+// of CYCLE planes, turns a plane's sum into the sum of the last W planes. With `pre` (the sum of this
+// cycle's planes) and, in slot j, the sum of the last cycle's planes j .. W - 1 before step j and this
+// cycle's plane j after it: about three additions a plane and W + 1 values held.
+template <int W, typename V>
+struct CcWindow {
+  static constexpr int CYCLE = W;
+  V ring[W], pre;
+  __device__ __forceinline__ void clear() {
+    pre = V(0);
 #pragma unroll
-  for (int ax = 0; ax < 3; ++ax) {
-    // the lower probe at pos - 0.5 clamps to the centre on the first voxel
-    const float hi = pos[ax] + 1 < len[ax] ? p[stride[ax]] : 0.0f;
-    const float lo = pos[ax] >= 1 ? p[-stride[ax]] : p[0];
-    half_diff[ax] = 0.5f * (hi - lo);
+    for (int j = 0; j < W; ++j) ring[j] = V(0);
   }
+  template <int J>
+  __device__ __forceinline__ V step(V plane) {
+    pre += plane;
+    V w = pre;
+    if constexpr (J + 1 < W) w += ring[J + 1];
+    ring[J] = plane;
+    if constexpr (J + 1 == W) {
 #pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    const int ax = pr.o[a][0] != 0.0f ? 0 : (pr.o[a][1] != 0.0f ? 1 : 2);
-    const float sgn = pr.o[a][ax];
-    const float h = ax == 0 ? half_diff[0] : (ax == 1 ? half_diff[1] : half_diff[2]);
-    // the upper probe of the last voxel lies at n - 0.5, outside the buffer
-    out[a] = pos[ax] >= len[ax] - 1 ? 0.0f : (sgn > 0.0f ? h : -h) * pr.inv_spacing[a];
+      for (int i = W - 2; i >= 1; --i) ring[i] += ring[i + 1];
+      pre = V(0);
+    }
+    return w;
   }
+};
+
+// Nine planes (radius 4) as three sums of three: four additions a plane and eight values held
+// (ten by the general scheme; the shorter cycle also keeps the code in the instruction cache).
+template <typename V>
+struct CcWindow<9, V> {
+  static constexpr int CYCLE = 6;
+  V last[2], three[6];  // by plane number modulo 2 and 6
+  __device__ __forceinline__ void clear() {
+    last[0] = last[1] = V(0);
+#pragma unroll
+    for (int j = 0; j < 6; ++j) three[j] = V(0);
+  }
+  template <int J>
+  __device__ __forceinline__ V step(V plane) {
+    const V s = (last[0] + last[1]) + plane;
+    last[J % 2] = plane;
+    const V w = (s + three[(J + 3) % 6]) + three[J];
+    three[J] = s;
+    return w;
+  }
+};
+
+// step(J, zin + J) for J = 0 .. CYCLE - 1, each with its own J at compile time.
+template <int CYCLE, int J = 0, typename Step>
+__device__ __forceinline__ void cc_cycle(Step& step, int zin) {
+  if constexpr (J < CYCLE) {
+    step(std::integral_constant<int, J>{}, zin + J);
+    cc_cycle<CYCLE, J + 1>(step, zin);
+  }
+}
+
+// 1 / v for normal v by the hardware's approximation and two Newton steps (within two units in the last
+// place; the IEEE division takes twice the instructions).
+__device__ __forceinline__ double reciprocal(double v) {
+  double r = __builtin_amdgcn_rcp(v);
+  r = fma(fma(-v, r, 1.0), r, r);
+  return fma(fma(-v, r, 1.0), r, r);
+}
+
+// sum / count by the count's reciprocal and one correction: exact where the quotient is (a window of
+// one value has that value as its mean, so its variance is zero, not a rounding error).
+__device__ __forceinline__ double mean_of(double sum, double count, double inv_count) {
+  const double q = sum * inv_count;
+  return fma(fma(-q, count, sum), inv_count, q);
 }
 
 __device__ float block_sum_f64(double v) {
@@ -95,54 +195,15 @@ __device__ float block_sum_f64(double v) {
   return (float)t;
 }
 
-// The split scale for an image bounded by `bound` (the host's cc_split_scale, on the device).
-__device__ __forceinline__ float cc_split_scale_dev(float bound) {
-  if (!(bound > 0.0f) || !isfinite(bound)) return 524288.0f;
-  int e = 0;
-  frexpf(bound, &e);  // bound < 2^e
-  return ldexpf(1.0f, 19 - e);
-}
-
-// One voxel's values split at the power-of-two step q = 1 / scale: v = h q + l with h an integer
-// (|h| <= 2^20 for |v| <= twice the bound) and l exact in f32 (|l| <= q / 2).
-struct CcSplit {
-  float h, l;
-};
-__device__ __forceinline__ CcSplit cc_split(float v, float scale, float step) {
-  const float h = rintf(v * scale);
-  return {h, v - h * step};
-}
-
-// The running sums of one column over the window's planes, for both images: the integer parts
-// (sums of h, h^2 and h_a h_b, exact in f64: at most 17^3 terms below 2^40) and the corrections of
-// the remainders (sums of l, l (2 h q + l) and h_a q l_b + l_a h_b q + l_a l_b), whose rounding is
-// relative to their own size (about q). A plane enters and one leaves per step; the integer parts
-// return exactly to zero with the values, so a window of zeros has zero sums up to the rounding of
-// the corrections (below 1e-19 for a bound of 1).
-struct CcColumn {
-  double e1a, e1b, e2a, e2b, e2ab;
-  double c1a, c1b, c2a, c2b, c2ab;
-};
-
-__device__ __forceinline__ void cc_column_step(CcColumn& col, const CcSplit& ea, const CcSplit& eb, const CcSplit& la,
-                                               const CcSplit& lb, float qa, float qb) {
-  const double hae = ea.h, hbe = eb.h, hal = la.h, hbl = lb.h;
-  col.e1a += hae - hal;
-  col.e1b += hbe - hbl;
-  col.e2a += fma(hae, hae, -hal * hal);
-  col.e2b += fma(hbe, hbe, -hbl * hbl);
-  col.e2ab += fma(hae, hbe, -hal * hbl);
-  const double lae = ea.l, lbe = eb.l, lal = la.l, lbl = lb.l;
-  const double Hae = hae * (double)qa, Hbe = hbe * (double)qb, Hal = hal * (double)qa, Hbl = hbl * (double)qb;
-  col.c1a += lae - lal;
-  col.c1b += lbe - lbl;
-  col.c2a += lae * (2.0 * Hae + lae) - lal * (2.0 * Hal + lal);
-  col.c2b += lbe * (2.0 * Hbe + lbe) - lbl * (2.0 * Hbl + lbl);
-  col.c2ab += fma(Hae, lbe, lae * (Hbe + lbe)) - fma(Hal, lbl, lal * (Hbl + lbl));
+// Waves per SIMD the registers are held to. At radius 4 the windows take 80 registers and the kernel
+// 187: held to 168 for three blocks a CU it spills 21 of them and takes 199 us at 1 mm for 156 us.
+template <int R>
+constexpr int cc_waves() {
+  return R <= 3 ? 3 : 2;
 }
 
 template <int R, bool MASKED, bool DIAGONAL>
-__global__ __launch_bounds__(cc_threads<R>()) void k_cc2(CcArgs a) {
+__global__ __launch_bounds__(kCcThreads, cc_waves<R>()) void k_cc2(CcArgs a) {
 #define FW_CC2_TILE xcd_block()
 #include "cc2_body.inc"
 #undef FW_CC2_TILE
@@ -152,7 +213,7 @@ __global__ __launch_bounds__(cc_threads<R>()) void k_cc2(CcArgs a) {
 // blocks are the blocks of its own launch (the same tiles, partials at the same indices of its
 // own partial buffers).
 template <int R, bool DIAGONAL>
-__global__ __launch_bounds__(cc_threads<R>()) void k_cc2_items(CcItems c) {
+__global__ __launch_bounds__(kCcThreads, cc_waves<R>()) void k_cc2_items(CcItems c) {
   constexpr bool MASKED = false;
   const unsigned gz = gridDim.z / (unsigned)c.count;
   const unsigned q = xcd_block().z / gz;
@@ -164,8 +225,8 @@ __global__ __launch_bounds__(cc_threads<R>()) void k_cc2_items(CcItems c) {
 
 template <int R, bool M>
 static void launch_cc_r(const CcArgs& a, hipStream_t s) {
-  if (a.probes.diagonal) launch((k_cc2<R, M, true>), cc_grid(a.d, a.tile_z), dim3(cc_threads<R>()), 0, s, a);
-  else launch((k_cc2<R, M, false>), cc_grid(a.d, a.tile_z), dim3(cc_threads<R>()), 0, s, a);
+  if (a.probes.diagonal) launch((k_cc2<R, M, true>), cc_grid(a.d, a.tile_z), dim3(kCcThreads), 0, s, a);
+  else launch((k_cc2<R, M, false>), cc_grid(a.d, a.tile_z), dim3(kCcThreads), 0, s, a);
 }
 
 template <int R>
@@ -173,8 +234,8 @@ static void launch_cc_items_r(const CcItems& c, hipStream_t s) {
   const CcArgs& a = c.a[0];
   dim3 g = cc_grid(a.d, a.tile_z);
   g.z *= (unsigned)c.count;
-  if (a.probes.diagonal) launch((k_cc2_items<R, true>), g, dim3(cc_threads<R>()), 0, s, c);
-  else launch((k_cc2_items<R, false>), g, dim3(cc_threads<R>()), 0, s, c);
+  if (a.probes.diagonal) launch((k_cc2_items<R, true>), g, dim3(kCcThreads), 0, s, c);
+  else launch((k_cc2_items<R, false>), g, dim3(kCcThreads), 0, s, c);
 }
 
 void launch_cc_items(const CcItems& c, hipStream_t s) {
@@ -202,15 +263,33 @@ dim3 cc_grid(const Dims& d, int tile_z) {
   return dim3((d.nx + kCcTX - 1) / kCcTX, (d.ny + kCcTY - 1) / kCcTY, (d.nz + tile_z - 1) / tile_z);
 }
 
-// The z run of a CC block: the longest of max_tile, max_tile / 2, ..., 1 planes whose grid still
-// has min_blocks blocks, so that a small level is not left to a few long-running blocks.
-int cc_tile_for(const Dims& d, int max_tile, int min_blocks) {
-  int t = std::max(1, max_tile);
-  for (; t > 1; t /= 2) {
-    const dim3 g = cc_grid(d, t);
-    if (size_t(g.x) * g.y * g.z >= size_t(std::max(1, min_blocks))) break;
+// The z run of a CC block. With a choice of the tuning table: the longest of max_tile, max_tile / 2,
+// ..., 1 planes whose grid still has min_blocks blocks. By default (max_tile 0) the run that takes
+// the least time: a block walks tile_z + 2R planes one after another, a CU holds two blocks (187
+// registers at radius 4), and a plane takes a pair of blocks kCcPairTime times a block alone (both
+// are bound by f64 arithmetic for most of it).
+constexpr double kCcPairTime = 1.5;
+int cc_tile_for(const Dims& d, int radius, int max_tile, int min_blocks) {
+  const long long tiles = (long long)((d.nx + kCcTX - 1) / kCcTX) * ((d.ny + kCcTY - 1) / kCcTY);
+  if (max_tile > 0) {
+    int t = max_tile;
+    for (; t > 1; t /= 2)
+      if (tiles * ((d.nz + t - 1) / t) >= std::max(1, min_blocks)) break;
+    return t;
   }
-  return t;
+  int best = d.nz;
+  double least = 1e300;
+  // at most kCcMostBlocks blocks, beyond one a tile
+  for (long long chunks = 1; chunks <= d.nz && (chunks == 1 || chunks * tiles <= kCcMostBlocks); ++chunks) {
+    const int t = (int)((d.nz + chunks - 1) / chunks);
+    const long long per_cu = (tiles * ((d.nz + t - 1) / t) + kCcCus - 1) / kCcCus;
+    const double time = double(t + 2 * radius) * (double(per_cu / 2) * kCcPairTime + double(per_cu % 2));
+    if (time < least) {
+      least = time;
+      best = t;
+    }
+  }
+  return best;
 }
 
 void launch_cc_pair(const CcArgs& a, hipStream_t s) {

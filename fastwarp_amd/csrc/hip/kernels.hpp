@@ -61,9 +61,6 @@ struct CcArgs {
   Dims d;
   int radius;
   int tile_z;
-  float scale_f, scale_m;  // 2^19 / (the image's bound rounded up to a power of two)
-  float step_f, step_m;    // 1 / scale
-  const float* bounds;     // device [2] (fixed, moving): when set, the scales come from these
   Probes probes;
   float* d_fixed;        // 3 planes: coefficient * grad(moving)
   float* d_moving;       // 3 planes: coefficient' * grad(fixed)
@@ -72,9 +69,12 @@ struct CcArgs {
 };
 void launch_cc_pair(const CcArgs& a, hipStream_t s);
 dim3 cc_grid(const Dims& d, int tile_z);
-// The longest z run of at most max_tile planes (halving) whose grid still has min_blocks blocks.
-int cc_tile_for(const Dims& d, int max_tile, int min_blocks = 512);
-constexpr int kCcTileZ = 16;  // the default longest z run
+// The planes a CC block walks: by default (max_tile 0) the split that takes the least time, else the
+// longest run of at most max_tile planes (halving) whose grid still has min_blocks blocks.
+int cc_tile_for(const Dims& d, int radius, int max_tile, int min_blocks);
+constexpr int kCcTileZ = 16, kCcMinBlocks = 512;  // where the table sets only the other knob
+constexpr long long kCcCus = 256, kCcMostBlocks = 8192;
+constexpr int kCcTileY = 8;  // a CC block's rows
 
 // --- per-block partial reductions ---
 // Largest |u/spacing| of two fields (b may be null) and sums of squares.

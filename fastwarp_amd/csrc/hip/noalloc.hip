@@ -1,7 +1,7 @@
 // fw_cc_pair_noalloc: the CC pair of fw_cc_pair on caller-owned device buffers, with no device or
-// host allocation. Its kernels keep their block partials and the two image bounds in `scratch`, a
-// static device array of fixed size (each GPU the library runs on holds its own copy until the
-// process ends). Host code never passes the array's name to a kernel: the name is a host-side
+// host allocation. Its kernels keep their block partials in `scratch`, a static device array of
+// fixed size (each GPU the library runs on holds its own copy until the process ends). Host code
+// never passes the array's name to a kernel: the name is a host-side
 // stand-in, and each device's address of its copy comes from hipGetSymbolAddress, taken once per
 // device with that device current and kept in `g_scratch`.
 //
@@ -29,64 +29,60 @@ void set_call_error(const std::string& message);
 namespace fw::hip {
 namespace {
 
-// The largest CC grid the scratch holds, in blocks of the CC kernel (64 x 8 x tile_z voxels): the
-// 1 mm grid (182 x 218 x 182) takes 1008 blocks.
-constexpr int kNoAllocMaxBlocks = 16384;
-// Blocks of the bound pass.
-constexpr int kBoundBlocks = 512;
-// Layout in 4-byte words: CC value partials (f32), CC counts (i32), bound partials (2 per block,
-// f32), then the two bounds.
+// The largest grid the entry point takes, in units of 64 x 8 x (at most 16) voxels (1 mm: 1,008).
+constexpr long long kNoAllocMaxUnits = 16384;
+// Every grid within that limit takes at most two CC blocks (32 x 8 voxels over a run of planes) a
+// unit: one for each half of a unit's columns where the run is at least the unit's, and by the
+// default rule at most kCcMostBlocks blocks where it is shorter.
+constexpr int kNoAllocMaxBlocks = 2 * int(kNoAllocMaxUnits);
+static_assert(kCcMostBlocks <= kNoAllocMaxBlocks, "the scratch holds every default z split");
+// Layout in 4-byte words: CC value partials (f32), CC counts (i32).
 constexpr size_t kOffCc = 0;
 constexpr size_t kOffCount = kOffCc + kNoAllocMaxBlocks;
-constexpr size_t kOffBoundPart = kOffCount + kNoAllocMaxBlocks;
-constexpr size_t kOffBounds = kOffBoundPart + 2 * kBoundBlocks;
-constexpr size_t kScratchWords = kOffBounds + 2;
+constexpr size_t kScratchWords = kOffCount + kNoAllocMaxBlocks;
 
-// 137,224 bytes per device.
+// 262,144 bytes per device.
 static __device__ __align__(256) uint32_t scratch[kScratchWords];
 
-// Per block: the largest finite |value| of each image (the bound fw_image_upload takes on the host).
-__global__ __launch_bounds__(256) void k_bound_partials(const float* __restrict__ f, const float* __restrict__ m, long long n,
-                                                        float* partial) {
-  float a = 0.0f, b = 0.0f;
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-    const float x = f[i], y = m[i];
-    if (isfinite(x)) a = fmaxf(a, fabsf(x));
-    if (isfinite(y)) b = fmaxf(b, fabsf(y));
-  }
-  const float ra = block_max(a);
-  const float rb = block_max(b);
-  if (threadIdx.x == 0) {
-    partial[2 * blockIdx.x] = ra;
-    partial[2 * blockIdx.x + 1] = rb;
-  }
-}
-
-__global__ __launch_bounds__(256) void k_bound_final(const float* __restrict__ partial, int blocks, float* bounds) {
-  float a = 0.0f, b = 0.0f;
-  for (int i = threadIdx.x; i < blocks; i += blockDim.x) {
-    a = fmaxf(a, partial[2 * i]);
-    b = fmaxf(b, partial[2 * i + 1]);
-  }
-  const float ra = block_max(a);
-  const float rb = block_max(b);
-  if (threadIdx.x == 0) {
-    bounds[0] = ra;
-    bounds[1] = rb;
+// The units of grid d: runs of 16 planes, halved while the grid has fewer than 512 units (grids of
+// 2^22 to 2^23 - 1 voxels: runs of 64, 256 units).
+long long noalloc_units(const Dims& d) {
+  const long long n = d.n();
+  const bool mid = n >= (1ll << 22) && n < (1ll << 23);
+  const long long columns = (long long)((d.nx + 63) / 64) * ((d.ny + 7) / 8);
+  for (int t = mid ? 64 : 16;; t /= 2) {
+    const long long units = columns * ((d.nz + t - 1) / t);
+    if (t == 1 || units >= (mid ? 256 : 512)) return units;
   }
 }
 
 // values[0] = values[1] = -(sum of the block partials) / (sum of the counts), the block partials
-// added in block order in f64 as fw_cc_pair adds them on the host.
-__global__ __launch_bounds__(64) void k_cc_value_final(const float* __restrict__ partial_cc, const int* __restrict__ count,
-                                                       int blocks, double* values) {
-  if (threadIdx.x != 0) return;
+// added in block order in f64 as fw_cc_pair adds them on the host: 256 threads stage them in LDS
+// (one thread loading them from memory itself took 30 us for 1,008 blocks), one adds them.
+__global__ __launch_bounds__(256) void k_cc_value_final(const float* __restrict__ partial_cc, const int* __restrict__ count,
+                                                        int blocks, double* values) {
+  constexpr int kStage = 2048;
+  __shared__ float cc[kStage];
+  __shared__ int cn[kStage];
   double total = 0.0;
   long long c = 0;
-  for (int b = 0; b < blocks; ++b) {
-    total += (double)partial_cc[b];
-    c += count[b];
+  for (int base = 0; base < blocks; base += kStage) {
+    const int m = min(kStage, blocks - base);
+    for (int b = threadIdx.x; b < m; b += blockDim.x) {
+      cc[b] = partial_cc[base + b];
+      cn[b] = count[base + b];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll 8
+      for (int b = 0; b < m; ++b) {
+        total += (double)cc[b];
+        c += cn[b];
+      }
+    }
+    __syncthreads();
   }
+  if (threadIdx.x != 0) return;
   const double v = c > 0 ? -total / (double)c : __builtin_nan("");
   values[0] = v;
   values[1] = v;
@@ -136,30 +132,22 @@ extern "C" int fw_cc_pair_noalloc(const fw_grid* grid, const float* fixed, const
     a.d = dims_of(g);
     a.radius = int(radius);
     // the same z runs as fw_cc_pair on a context with the default table, so the same bits
-    const uint64_t nv = uint64_t(a.d.n());
-    a.tile_z = cc_tile_for(a.d, int(default_tuning().get("cc.tile_z", nv, kCcTileZ)),
-                           int(default_tuning().get("cc.min_blocks", nv, 512)));
+    a.tile_z = cc_tile(default_tuning(), a.d, a.radius);
     const dim3 gr = cc_grid(a.d, a.tile_z);
     const long long blocks = (long long)gr.x * gr.y * gr.z;
-    if (blocks > kNoAllocMaxBlocks)
-      fw::invalid("cc noalloc", "the grid needs " + std::to_string(blocks) + " CC blocks, more than the " +
-                                    std::to_string(kNoAllocMaxBlocks) + " the static scratch holds");
+    const long long units = noalloc_units(a.d);
+    if (units > kNoAllocMaxUnits || blocks > kNoAllocMaxBlocks)
+      fw::invalid("cc noalloc", "the grid has " + std::to_string(units) + " units of 64 x 8 x 16 voxels, more than the " +
+                                    std::to_string(kNoAllocMaxUnits) + " the static scratch holds");
     uint32_t* ptr = scratch_of_current_device();
     a.probes = probes_of(g);
     a.d_fixed = d_fixed;
     a.d_moving = d_moving;
     a.partial_cc = reinterpret_cast<float*>(ptr + kOffCc);
     a.partial_count = reinterpret_cast<int*>(ptr + kOffCount);
-    a.bounds = reinterpret_cast<const float*>(ptr + kOffBounds);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const long long n = a.d.n();
-    float* bound_part = reinterpret_cast<float*>(ptr + kOffBoundPart);
-    float* bounds = reinterpret_cast<float*>(ptr + kOffBounds);
-    const int bb = int(std::min<long long>(kBoundBlocks, std::max<long long>(1, (n + 255) / 256)));
-    launch(k_bound_partials, dim3(bb), dim3(256), 0, s, fixed, moving, n, bound_part);
-    launch(k_bound_final, dim3(1), dim3(256), 0, s, (const float*)bound_part, bb, bounds);
     launch_cc_pair(a, s);
-    launch(k_cc_value_final, dim3(1), dim3(64), 0, s, (const float*)a.partial_cc, (const int*)a.partial_count, int(blocks),
+    launch(k_cc_value_final, dim3(1), dim3(256), 0, s, (const float*)a.partial_cc, (const int*)a.partial_count, int(blocks),
            values);
     if (hipGetLastError() != hipSuccess) throw std::runtime_error("fw_cc_pair_noalloc: kernel launch failed");
     return FW_OK;

@@ -160,8 +160,8 @@ int fw_cc_pair(fw_ctx* ctx, const fw_image* fixed, const fw_image* moving, const
  * three planes each, written), values (2 f64, written: values[0] = values[1], as fw_cc_pair's).
  * The work is enqueued on `stream` (a hipStream_t, NULL for the null stream) and the call returns
  * without waiting; nothing is allocated. Block partials live in a static per-device scratch of
- * 137,224 bytes, which limits the grid to 16,384 CC blocks of 64 x 8 x (at most 16) voxels (the
- * 1 mm grid needs 1008); a larger grid is rejected with FW_ERR_INVALID. Calls that overlap on one
+ * 262,144 bytes, which limits the grid to 16,384 units of 64 x 8 x (at most 16) voxels (the
+ * 1 mm grid has 1008); a larger grid is rejected with FW_ERR_INVALID. Calls that overlap on one
  * GPU race on that scratch. Results are the same bits as fw_cc_pair's on the same images. Errors:
  * the status, and fw_last_error(NULL) for the text. */
 int fw_cc_pair_noalloc(const fw_grid* grid, const float* fixed, const float* moving, uint32_t radius, float* d_fixed,
