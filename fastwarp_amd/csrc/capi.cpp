@@ -165,8 +165,7 @@ int fw_image_download(fw_ctx* ctx, const fw_image* image, double* out) {
   return guard(ctx, [&] {
     need(image, "image");
     need(out, "output");
-    fw::Image v = ctx->backend.download_image(image->h);
-    std::memcpy(out, v.data.data(), v.data.size() * sizeof(double));
+    ctx->backend.download_image_to(image->h, out);
   });
 }
 
@@ -208,9 +207,7 @@ int fw_field_download(fw_ctx* ctx, const fw_field* field, double* aos) {
   return guard(ctx, [&] {
     need(field, "field");
     need(aos, "output");
-    fw::VectorField v = ctx->backend.download_field(field->h);
-    for (size_t i = 0; i < v.data.size(); ++i)
-      for (int c = 0; c < 3; ++c) aos[3 * i + c] = v.data[i][c];
+    ctx->backend.download_field_to(field->h, aos);
   });
 }
 

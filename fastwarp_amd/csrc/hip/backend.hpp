@@ -273,7 +273,7 @@ class HipBackend {
   // floor((n - 1) * spacing / mm + 1e-9) + 1 voxels per axis), trilinear from the source indices
   // min(i * mm / spacing, n - 1); a copy when every axis already has spacing mm (within 1e-6).
   HImage resample_isotropic(const HImage& im, double mm);
-  Image download_image(const HImage& im);
+  void download_image_to(const HImage& im, double* out);
   HField zero_field(const Grid& g);
   HField upload_field(const VectorField& f);
   VectorField download_field(const HField& f);
