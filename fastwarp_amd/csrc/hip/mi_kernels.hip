@@ -7,6 +7,8 @@
 // same bits whatever the block count or scheduling. The host finishes it in f64.
 // Parameter derivatives of the linear stage accumulate in FP64 per thread and reduce per block in
 // a fixed tree; the host adds the block partials in block order.
+#include <algorithm>
+
 #include "device_common.hpp"
 #include "mi_kernels.hpp"
 
@@ -44,6 +46,39 @@ __device__ __forceinline__ unsigned long long to_fixed(float w) {
 __device__ __forceinline__ int clamp_bin(float term, int bins) {
   int b = (int)term;  // truncation toward zero, as the reference's `as i64`
   return b < 2 ? 2 : (b > bins - 3 ? bins - 3 : b);
+}
+
+// tri() for an image below 2^30 voxels: the corners as 32-bit byte offsets beside the image's scalar
+// address, all eight loads issued before the first blend (left to itself the compiler puts the x
+// neighbours' loads behind a branch on their weight). The same blends, so the same bits.
+__device__ __forceinline__ float tri32(const float* __restrict__ img, const Dims& d, float cx, float cy, float cz) {
+  int bx, by, bz;
+  float wx, wy, wz;
+  axis_weight(cx, d.nx, bx, wx);
+  axis_weight(cy, d.ny, by, wy);
+  axis_weight(cz, d.nz, bz, wz);
+  const unsigned row = 4u * (unsigned)d.nx, plane = row * (unsigned)d.ny;
+  const unsigned sx = bx + 1 < d.nx ? 4u : 0u, sy = by + 1 < d.ny ? row : 0u, sz = bz + 1 < d.nz ? plane : 0u;
+  const unsigned o0 = 4u * (unsigned)bx + row * (unsigned)by + plane * (unsigned)bz;
+  const unsigned o2 = o0 + sy, o4 = o0 + sz, o6 = o2 + sz;
+  const char* p = reinterpret_cast<const char*>(img);
+  auto at = [p](unsigned o) __attribute__((always_inline)) { return *reinterpret_cast<const float*>(p + o); };
+  float v0 = at(o0), v1 = at(o0 + sx), v2 = at(o2), v3 = at(o2 + sx);
+  float v4 = at(o4), v5 = at(o4 + sx), v6 = at(o6), v7 = at(o6 + sx);
+  asm("" : "+v"(v0), "+v"(v1), "+v"(v2), "+v"(v3), "+v"(v4), "+v"(v5), "+v"(v6), "+v"(v7));
+  const float r00 = wx > 0.0f ? v0 + (v1 - v0) * wx : v0;
+  const float r01 = wx > 0.0f ? v2 + (v3 - v2) * wx : v2;
+  const float r10 = wx > 0.0f ? v4 + (v5 - v4) * wx : v4;
+  const float r11 = wx > 0.0f ? v6 + (v7 - v6) * wx : v6;
+  const float p0 = wy > 0.0f ? r00 + (r01 - r00) * wy : r00;
+  const float p1 = wy > 0.0f ? r10 + (r11 - r10) * wy : r10;
+  return wz > 0.0f ? p0 + (p1 - p0) * wz : p0;
+}
+
+template <bool WIDE>
+__device__ __forceinline__ float sample_tri(const float* __restrict__ img, const Dims& d, float cx, float cy, float cz) {
+  if constexpr (WIDE) return tri(img, d, cx, cy, cz);
+  else return tri32(img, d, cx, cy, cz);
 }
 
 // Central difference along physical axis `a` at a continuous index (interp.rs:102-121).
@@ -158,20 +193,59 @@ struct SampleEval {
   float term, cx, cy, cz;
 };
 
-__device__ __forceinline__ SampleEval eval_sample(const MiSampledArgs& a, float4 s) {
+// The map of one transform: the moving image's continuous index of a sample (A s + b).
+struct SampleMap {
+  const float* a;
+  const float* b;
+};
+
+template <bool WIDE>
+__device__ __forceinline__ SampleEval eval_sample(const MiSampledArgs& a, const SampleMap& t, float4 s) {
   SampleEval e;
   e.ok = false;
   e.fbin = __float_as_int(s.w);
-  e.cx = fmaf(a.a[0], s.x, fmaf(a.a[1], s.y, fmaf(a.a[2], s.z, a.b[0])));
-  e.cy = fmaf(a.a[3], s.x, fmaf(a.a[4], s.y, fmaf(a.a[5], s.z, a.b[1])));
-  e.cz = fmaf(a.a[6], s.x, fmaf(a.a[7], s.y, fmaf(a.a[8], s.z, a.b[2])));
+  e.cx = fmaf(t.a[0], s.x, fmaf(t.a[1], s.y, fmaf(t.a[2], s.z, t.b[0])));
+  e.cy = fmaf(t.a[3], s.x, fmaf(t.a[4], s.y, fmaf(t.a[5], s.z, t.b[1])));
+  e.cz = fmaf(t.a[6], s.x, fmaf(t.a[7], s.y, fmaf(t.a[8], s.z, t.b[2])));
   if (!inside(a.md, e.cx, e.cy, e.cz)) return e;
-  const float mv = tri(a.moving, a.md, e.cx, e.cy, e.cz);
+  const float mv = sample_tri<WIDE>(a.moving, a.md, e.cx, e.cy, e.cz);
   if (!(mv >= a.moving_min && mv <= a.moving_max)) return e;  // also rejects NaN
   e.term = (mv - a.moving_min) * a.inv_bin_size + 2.0f;
   e.mbin = clamp_bin(e.term, a.bins);
   e.ok = true;
   return e;
+}
+
+// A weight below one in 2^-32 fixed point, as to_fixed gives it.
+__device__ __forceinline__ unsigned long long to_fixed_below_one(float w) {
+  return (unsigned long long)(unsigned)rintf(w * 4294967296.0f);
+}
+
+// Adds one sample to a block histogram h (bins x bins joint cells, then the fixed marginal). The four
+// weights' arguments lie in [1, 2], [0, 1], [0, 1] and [1, 2], where each is one of the kernel's two
+// polynomials (both give the same bits at 1, and zero at 2), unless the value lies a rounding above
+// the top of the range: then each argument picks its own.
+__device__ __forceinline__ void bin_sample(unsigned long long* h, int bins, const SampleEval& e) {
+  unsigned long long* row = h + __mul24(e.fbin, bins) + e.mbin;
+  atomicAdd(&h[__mul24(bins, bins) + e.fbin], 1ull);
+  const float m = (float)e.mbin;
+  if (e.term - m <= 1.0f) {
+    auto near = [](float a) { const float s = a * a; return (4.0f - 6.0f * s + 3.0f * s * a) * (1.0f / 6.0f); };
+    auto far = [](float a) { const float s = a * a; return (8.0f - 12.0f * a + 6.0f * s - s * a) * (1.0f / 6.0f); };
+    const float w0 = far(fabsf((float)(e.mbin - 1) - e.term)), w1 = near(fabsf(m - e.term));
+    const float w2 = near(fabsf((float)(e.mbin + 1) - e.term)), w3 = far(fabsf((float)(e.mbin + 2) - e.term));
+    // a weight that rounding leaves below zero counts as none
+    atomicAdd(&row[-1], to_fixed_below_one(fmaxf(w0, 0.0f)));
+    atomicAdd(&row[0], to_fixed_below_one(w1));
+    atomicAdd(&row[1], to_fixed_below_one(w2));
+    atomicAdd(&row[2], to_fixed_below_one(fmaxf(w3, 0.0f)));
+    return;
+  }
+#pragma unroll
+  for (int q = -1; q <= 2; ++q) {
+    const float w = bspline3((float)(e.mbin + q) - e.term);
+    if (w > 0.0f) atomicAdd(&row[q], to_fixed(w));
+  }
 }
 
 }  // namespace
@@ -200,78 +274,75 @@ int mi_deriv_blocks(int count, int cap) {
   return b < 1 ? 1 : (b > c ? c : b);
 }
 
-// The block's histogram (LDS, 64-bit atomics) is written to its own slot of `hist_slots`; a second
-// kernel adds the slots, so the global histogram needs neither clearing nor global atomics.
-__global__ __launch_bounds__(1024) void k_mi_sampled_hist(MiSampledArgs a) {
-  extern __shared__ unsigned long long h[];
-  const int bins = a.bins;
-  const int cells = bins * bins + bins;
-  for (int i = threadIdx.x; i < cells + 1; i += blockDim.x) h[i] = 0ull;
-  __syncthreads();
-  unsigned int mine = 0;
-  const SampleRange rg = sample_range(a.count);
-  for (int s = rg.lo + threadIdx.x; s < rg.hi; s += blockDim.x) {
-    const SampleEval e = eval_sample(a, a.samples[s]);
-    if (!e.ok) continue;
-    ++mine;
-    atomicAdd(&h[bins * bins + e.fbin], 1ull);
-    unsigned long long* row = h + e.fbin * bins;
-#pragma unroll
-    for (int q = -1; q <= 2; ++q) {
-      const int m = e.mbin + q;
-      const float w = bspline3((float)m - e.term);
-      if (w > 0.0f) atomicAdd(&row[m], to_fixed(w));
+// The maps of a pass's transforms, as a kernel argument of no more than they take (the single pass's
+// map is in its MiSampledArgs).
+template <int K>
+struct HistMaps {
+  float a[K][9], b[K][3];
+  explicit HistMaps(const MiBatch& m) {
+    for (int k = 0; k < K; ++k) {
+      for (int q = 0; q < 9; ++q) a[k][q] = m.a[k][q];
+      for (int q = 0; q < 3; ++q) b[k][q] = m.b[k][q];
     }
   }
-  if (mine) atomicAdd(&h[cells], (unsigned long long)mine);
-  __syncthreads();
-  unsigned long long* slot = a.hist_slots + (size_t)blockIdx.x * (cells + 1);
-  for (int i = threadIdx.x; i < cells + 1; i += blockDim.x) slot[i] = h[i];
-}
+  __device__ __forceinline__ SampleMap of(const MiSampledArgs&, int k) const { return SampleMap{a[k], b[k]}; }
+};
+template <>
+struct HistMaps<1> {
+  explicit HistMaps(const MiBatch&) {}
+  __device__ __forceinline__ SampleMap of(const MiSampledArgs& s, int) const { return SampleMap{s.a, s.b}; }
+};
 
-// K transforms per pass: each sample record is read once and binned under every transform, into
-// the K histograms of the block's LDS (the samples, the anchor and the moving image are shared).
-template <int K>
-__global__ __launch_bounds__(1024) void k_mi_sampled_hist_batch(MiSampledArgs a, MiBatch batch) {
+// K transforms per pass over the same samples, each with its own histogram in the block's LDS (64-bit
+// atomics) and its own K-th of the block's threads, so that the transforms' gathers and atomics run
+// beside each other (one after another in every thread, a pass of four took 17.6 us on 3,267 samples
+// and 38 on 225,658, for 7.0 and 11.4 of one). A block writes its histograms to its own slot of
+// `hist_slots`; a second kernel adds the slots, so the global histogram needs neither clearing nor
+// global atomics. With COPIES > 1 the lanes take turns over that many copies of the histogram, added
+// as the slot is written: most samples of a volume with background fall into a few cells, and the
+// additions of one wave to one cell are done one by one.
+template <int K, int COPIES, bool WIDE>
+__global__ __launch_bounds__(1024) void k_mi_sampled_hist(MiSampledArgs a, HistMaps<K> batch) {
   extern __shared__ unsigned long long h[];
   const int bins = a.bins;
   const int cells = bins * bins + bins;
   const int C = cells + 1;
-  for (int i = threadIdx.x; i < K * C; i += blockDim.x) h[i] = 0ull;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < K * COPIES * C; i += blockDim.x) h[i] = 0ull;
   __syncthreads();
-  unsigned int mine[K];
-#pragma unroll
-  for (int k = 0; k < K; ++k) mine[k] = 0;
+  const int group = (int)blockDim.x / K;
+  const int k = K == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / group);
+  const SampleMap map = batch.of(a, k);
+  unsigned long long* mine = h + (k * COPIES + (COPIES == 1 ? 0 : (int)(threadIdx.x % COPIES))) * C;
+  unsigned int valid = 0;
   const SampleRange rg = sample_range(a.count);
-  for (int s = rg.lo + threadIdx.x; s < rg.hi; s += blockDim.x) {
-    const float4 smp = a.samples[s];
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      MiSampledArgs ak = a;
-#pragma unroll
-      for (int q = 0; q < 9; ++q) ak.a[q] = batch.a[k][q];
-#pragma unroll
-      for (int q = 0; q < 3; ++q) ak.b[q] = batch.b[k][q];
-      const SampleEval e = eval_sample(ak, smp);
-      if (!e.ok) continue;
-      ++mine[k];
-      unsigned long long* hk = h + k * C;
-      atomicAdd(&hk[bins * bins + e.fbin], 1ull);
-      unsigned long long* row = hk + e.fbin * bins;
-#pragma unroll
-      for (int q = -1; q <= 2; ++q) {
-        const int m = e.mbin + q;
-        const float w = bspline3((float)m - e.term);
-        if (w > 0.0f) atomicAdd(&row[m], to_fixed(w));
-      }
-    }
+  int s = rg.lo + ((int)threadIdx.x - k * group);
+  float4 next = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (s < rg.hi) next = a.samples[s];
+  while (s < rg.hi) {
+    const float4 smp = next;
+    s += group;
+    if (s < rg.hi) next = a.samples[s];  // in flight while this sample is binned
+    const SampleEval e = eval_sample<WIDE>(a, map, smp);
+    if (!e.ok) continue;
+    ++valid;
+    bin_sample(mine, bins, e);
   }
-#pragma unroll
-  for (int k = 0; k < K; ++k)
-    if (mine[k]) atomicAdd(&h[k * C + cells], (unsigned long long)mine[k]);
+  if (valid) atomicAdd(&mine[cells], (unsigned long long)valid);
   __syncthreads();
   unsigned long long* slot = a.hist_slots + (size_t)blockIdx.x * K * C;
-  for (int i = threadIdx.x; i < K * C; i += blockDim.x) slot[i] = h[i];
+#pragma unroll 4
+  for (int i = threadIdx.x; i < K * C; i += blockDim.x) {
+    if constexpr (COPIES == 1) {
+      slot[i] = h[i];
+    } else {
+      static_assert(COPIES == 1 || K == 1, "copies are for the single pass");
+      unsigned long long t = 0ull;
+#pragma unroll
+      for (int q = 0; q < COPIES; ++q) t += h[q * C + i];
+      slot[i] = t;
+    }
+  }
 }
 
 int mi_batch_capacity(int bins) {
@@ -280,20 +351,37 @@ int mi_batch_capacity(int bins) {
   return int(fit < 1 ? 1 : (fit > size_t(kMiMaxBatch) ? kMiMaxBatch : fit));
 }
 
+// Images whose byte offsets do not fit 32 bits take the 64-bit form of the gathers.
+static bool wide_image(const MiSampledArgs& a) { return a.md.n() >= (1ll << 30); }
+
+// Blocks of at least this many samples keep copies of their histogram.
+constexpr int kMiCopies = 4;
+constexpr int kMiCopySamples = 2048;
+
+template <int K, int COPIES>
+static void launch_hist(const MiSampledArgs& a, const MiBatch& batch, int blocks, hipStream_t s) {
+  const size_t lds = size_t(K) * COPIES * size_t(a.bins * a.bins + a.bins + 1) * sizeof(unsigned long long);
+  // a batch's threads: as many a transform as the single pass has, up to 1,024 in all
+  const int one = a.threads > 0 ? a.threads : mi_sampled_threads(a.count);
+  const dim3 t(K * std::min(one, K == 1 ? 1024 : (K == 2 ? 512 : 256)));
+  if (wide_image(a)) launch((k_mi_sampled_hist<K, COPIES, true>), dim3(blocks), t, (uint32_t)lds, s, a, HistMaps<K>(batch));
+  else launch((k_mi_sampled_hist<K, COPIES, false>), dim3(blocks), t, (uint32_t)lds, s, a, HistMaps<K>(batch));
+}
+
 void launch_mi_sampled_hist_batch(const MiSampledArgs& a, const MiBatch& batch, int count, int blocks, hipStream_t s) {
-  const size_t lds = size_t(count) * size_t(a.bins * a.bins + a.bins + 1) * sizeof(unsigned long long);
-  const dim3 t(a.threads > 0 ? a.threads : mi_sampled_threads(a.count));
   switch (count) {
-    case 2: launch(k_mi_sampled_hist_batch<2>, dim3(blocks), t, (uint32_t)lds, s, a, batch); break;
-    case 3: launch(k_mi_sampled_hist_batch<3>, dim3(blocks), t, (uint32_t)lds, s, a, batch); break;
-    case 4: launch(k_mi_sampled_hist_batch<4>, dim3(blocks), t, (uint32_t)lds, s, a, batch); break;
+    case 2: launch_hist<2, 1>(a, batch, blocks, s); break;
+    case 3: launch_hist<3, 1>(a, batch, blocks, s); break;
+    case 4: launch_hist<4, 1>(a, batch, blocks, s); break;
     default: break;
   }
 }
 
 void launch_mi_sampled_hist(const MiSampledArgs& a, int blocks, hipStream_t s) {
-  const size_t lds = size_t(a.bins * a.bins + a.bins + 1) * sizeof(unsigned long long);
-  launch(k_mi_sampled_hist, dim3(blocks), dim3(a.threads > 0 ? a.threads : mi_sampled_threads(a.count)), lds, s, a);
+  const MiBatch none{};
+  const size_t lds = kMiCopies * size_t(a.bins * a.bins + a.bins + 1) * sizeof(unsigned long long);
+  if (a.count / blocks >= kMiCopySamples && lds <= (size_t(64) << 10)) launch_hist<1, kMiCopies>(a, none, blocks, s);
+  else launch_hist<1, 1>(a, none, blocks, s);
 }
 
 // hist[c] = sum of the slots' cell c, for every cell and the valid count. A block of 16 waves
@@ -479,6 +567,7 @@ void launch_mi_sum_finish(const unsigned long long* slots, int nslots, int count
 
 // Per sample: sum_k B3'(k - term) * ratio[f, k] * (grad M . dT/dtheta_p) for every parameter
 // (mi.rs:405-433 with the ratio weights of :752-757), accumulated in FP64.
+template <bool WIDE>
 __global__ __launch_bounds__(256) void k_mi_sampled_deriv(MiSampledArgs a) {
   __shared__ float ratio[kMiMaxBins * kMiMaxBins];
   __shared__ double red[4 * 12];
@@ -491,7 +580,7 @@ __global__ __launch_bounds__(256) void k_mi_sampled_deriv(MiSampledArgs a) {
   const SampleRange rg = sample_range(a.count);
   for (int s = rg.lo + threadIdx.x; s < rg.hi; s += blockDim.x) {
     const float4 smp = a.samples[s];
-    const SampleEval e = eval_sample(a, smp);
+    const SampleEval e = eval_sample<WIDE>(a, SampleMap{a.a, a.b}, smp);
     if (!e.ok) continue;
     float w = 0.0f;
 #pragma unroll
@@ -555,7 +644,8 @@ __global__ __launch_bounds__(256) void k_mi_sampled_deriv(MiSampledArgs a) {
 }
 
 void launch_mi_sampled_deriv(const MiSampledArgs& a, int blocks, hipStream_t s) {
-  launch(k_mi_sampled_deriv, dim3(blocks), dim3(256), 0, s, a);
+  if (wide_image(a)) launch(k_mi_sampled_deriv<true>, dim3(blocks), dim3(256), 0, s, a);
+  else launch(k_mi_sampled_deriv<false>, dim3(blocks), dim3(256), 0, s, a);
 }
 
 // out[k] = sum over the blocks of partial[b * 12 + k], k < np, in a fixed order: 16 waves take
