@@ -54,10 +54,10 @@ DeviceContext::~DeviceContext() {
   release_idle();
   for (auto& s : scratch_)
     if (s.p) hipFree(s.p);
-  if (pinned_) hipHostFree(pinned_);
+  if (pinned_.p) hipHostFree(pinned_.p);
   if (mailbox_) hipHostFree(mailbox_);
   for (auto& m : mapped_)
-    if (m.host) hipHostFree(m.host);
+    if (m.host.p) hipHostFree(m.host.p);
   for (auto& c : stage_) hipHostFree(c.p);
   for (auto& kv : taps_) hipFree(kv.second.first);
   for (auto& s : spans_) {
@@ -66,8 +66,6 @@ DeviceContext::~DeviceContext() {
   }
   (void)hipStreamDestroy(stream_);
 }
-
-static size_t round_bytes(size_t b) { return (b + 255) & ~size_t(255); }
 
 void* DeviceContext::acquire(size_t bytes) {
   bytes = round_bytes(std::max<size_t>(bytes, 256));
@@ -111,40 +109,55 @@ void DeviceContext::release_idle() {
 }
 
 void* DeviceContext::scratch(int slot, size_t bytes) {
-  Scratch& s = scratch_[slot];
-  if (s.bytes < bytes) {
-    if (s.p) {
-      hipStreamSynchronize(stream_);
-      hipFree(s.p);
-    }
-    s.bytes = round_bytes(bytes * 2);
-    check(hipMalloc(&s.p, s.bytes), "hipMalloc scratch");
-  }
-  return s.p;
+  void* p = grow(
+      scratch_[slot], bytes,
+      [&](size_t want) -> void* {
+        void* q = nullptr;
+        if (hipMalloc(&q, want) == hipSuccess) return q;
+        (void)hipGetLastError();
+        return nullptr;
+      },
+      [&](void* old) {
+        hipStreamSynchronize(stream_);
+        hipFree(old);
+      });
+  if (!p && bytes > 0) throw Error("hip", "scratch allocation of " + std::to_string(bytes) + " bytes failed");
+  return p;
+}
+
+// Host memory of the given flags, or nullptr (the error is taken from the runtime).
+static void* host_malloc(size_t bytes, unsigned flags) {
+  void* p = nullptr;
+  if (hipHostMalloc(&p, bytes, flags) == hipSuccess) return p;
+  (void)hipGetLastError();
+  return nullptr;
 }
 
 void* DeviceContext::pinned(size_t bytes) {
-  if (pinned_bytes_ < bytes) {
-    if (pinned_) hipHostFree(pinned_);
-    pinned_bytes_ = round_bytes(bytes * 2);
-    check(hipHostMalloc(&pinned_, pinned_bytes_, hipHostMallocDefault), "hipHostMalloc");
-  }
-  return pinned_;
+  void* p = grow(
+      pinned_, bytes, [](size_t want) { return host_malloc(want, hipHostMallocDefault); }, [](void* old) { hipHostFree(old); });
+  if (!p && bytes > 0) throw Error("hip", "pinned allocation of " + std::to_string(bytes) + " bytes failed");
+  return p;
 }
 
 void* DeviceContext::mapped(int slot, size_t bytes, void** device) {
   Mapped& m = mapped_[slot];
-  if (m.bytes < bytes) {
-    if (m.host) {
-      sync();
-      hipHostFree(m.host);
+  if (m.host.bytes < bytes) {
+    if (m.host.p) sync();
+    m.dev = nullptr;
+    if (!grow(
+            m.host, bytes, [](size_t want) { return host_malloc(want, hipHostMallocMapped | hipHostMallocCoherent); },
+            [](void* old) { hipHostFree(old); }))
+      throw Error("hip", "mapped allocation of " + std::to_string(bytes) + " bytes failed");
+    if (hipHostGetDevicePointer(&m.dev, m.host.p, 0) != hipSuccess) {
+      (void)hipGetLastError();
+      hipHostFree(m.host.p);
+      m = Mapped{};
+      throw Error("hip", "no device address for mapped host memory");
     }
-    m.bytes = round_bytes(bytes * 2);
-    check(hipHostMalloc(&m.host, m.bytes, hipHostMallocMapped | hipHostMallocCoherent), "hipHostMalloc mapped");
-    check(hipHostGetDevicePointer(&m.dev, m.host, 0), "hipHostGetDevicePointer");
   }
   *device = m.dev;
-  return m.host;
+  return m.host.p;
 }
 
 void* DeviceContext::stage(size_t bytes) {

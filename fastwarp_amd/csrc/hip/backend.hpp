@@ -21,6 +21,7 @@
 #include "../host/backend_types.hpp"
 #include "../host/tuning.hpp"
 #include "../host/grid.hpp"
+#include "../host/grow.hpp"
 #include "../host/mi_host.hpp"
 #include "../host/pyramid.hpp"
 #include "../host/transform.hpp"
@@ -107,21 +108,16 @@ class DeviceContext : public HostSpanSink {
   hipStream_t stream_{};
   std::map<size_t, std::vector<void*>> free_;
   uint64_t held_ = 0, peak_ = 0;
-  struct Scratch {
-    void* p = nullptr;
-    size_t bytes = 0;
-  };
-  Scratch scratch_[10];
-  void* pinned_ = nullptr;
+  GrowBuffer scratch_[10];
+  GrowBuffer pinned_;
   struct StageChunk {
     char* p = nullptr;
     size_t capacity = 0, used = 0;
   };
   std::vector<StageChunk> stage_;
   struct Mapped {
-    void* host = nullptr;
+    GrowBuffer host;
     void* dev = nullptr;
-    size_t bytes = 0;
   };
   Mapped mapped_[8];
   static constexpr int kDoneBase = 64;  // words 0..63: the inversion's progress and stop words
@@ -129,7 +125,6 @@ class DeviceContext : public HostSpanSink {
   uint32_t* mailbox_ = nullptr;
   uint32_t* mailbox_dev_ = nullptr;
   uint32_t tag_ = 0;
-  size_t pinned_bytes_ = 0;
   std::map<std::pair<double, size_t>, std::pair<void*, int>> taps_;
   std::map<std::pair<double, size_t>, std::vector<double>> host_taps_;
   bool profiling_ = false;

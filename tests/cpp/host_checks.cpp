@@ -19,6 +19,7 @@
 #include "../../fastwarp_amd/csrc/hip/fastdiv.hpp"
 #include "../../fastwarp_amd/csrc/host/admission.hpp"
 #include "../../fastwarp_amd/csrc/host/gauss_taps.hpp"
+#include "../../fastwarp_amd/csrc/host/grow.hpp"
 #include "../../fastwarp_amd/csrc/host/hdf5.hpp"
 #include "../../fastwarp_amd/csrc/host/itk_h5.hpp"
 #include "../../fastwarp_amd/csrc/host/linear.hpp"
@@ -1033,7 +1034,36 @@ static void host_loops() {
   ok("host_loops");
 }
 
+// A growable buffer whose replacement fails: the old buffer is gone, so no later request, however
+// small, may be given it again; and where only twice the request is too much, the request is met.
+static void grow_buffer() {
+  char memory[4096];
+  size_t limit = sizeof(memory), used = 0;
+  int live = 0;
+  auto alloc = [&](size_t bytes) -> void* {
+    if (bytes > limit || used + bytes > sizeof(memory)) return nullptr;
+    void* p = memory + used;
+    used += bytes;
+    ++live;
+    return p;
+  };
+  auto release = [&](void*) { --live; };
+  GrowBuffer b;
+  CHECK(grow(b, 0, alloc, release) == nullptr && live == 0, "no buffer for nothing");
+  void* first = grow(b, 256, alloc, release);
+  CHECK(first == memory && b.bytes == 512 && live == 1, "twice the first request");
+  CHECK(grow(b, 512, alloc, release) == first && grow(b, 1, alloc, release) == first, "a request that fits keeps the buffer");
+  limit = 0;
+  CHECK(grow(b, 1024, alloc, release) == nullptr && live == 0, "a failed replacement");
+  CHECK(grow(b, 64, alloc, release) == nullptr && grow(b, 512, alloc, release) == nullptr, "the released buffer is not given out again");
+  limit = 1100;
+  void* exact = grow(b, 1024, alloc, release);
+  CHECK(exact == memory + 512 && b.bytes == 1024 && live == 1, "the request alone where twice it fails");
+  ok("grow_buffer");
+}
+
 int main() {
+  grow_buffer();
   host_loops();
   mt19937();
   regular_sampling();
