@@ -423,16 +423,33 @@ HImage HipBackend::upload_image_f32(const Grid& g, const float* data) {
   return im;
 }
 
-// Through pinned memory and the host threads: a copy into pageable memory and the zero-filled vectors
-// between it and the caller's array took 66 ms for a 1 mm field, this way takes about 6.
+// C planes of n values each, interleaved into the caller's f64 array through pinned memory and the host
+// threads: a copy into pageable memory and the zero-filled vectors between it and the caller's array took
+// 66 ms for a 1 mm field, this way takes about 6. Pieces of at most kDownloadFloats values bound the
+// pinned memory that a download takes and the context keeps, whatever the volume. A 1 mm field (22 M
+// values) is one piece: cut into three, its download took 0.8 ms more.
+template <size_t C>
+static void download_planes(DeviceContext& ctx, const float* src, size_t n, double* out, const char* what) {
+  constexpr size_t kDownloadFloats = size_t(1) << 25;
+  const size_t piece = std::min(n, kDownloadFloats / C);
+  auto* stage = static_cast<float*>(ctx.pinned(C * piece * sizeof(float)));
+  for (size_t begin = 0; begin < n; begin += piece) {
+    const size_t m = std::min(piece, n - begin);
+    // the planes of a whole volume follow each other: one copy
+    const size_t copies = m == n ? 1 : C, values = m == n ? C * n : m;
+    for (size_t c = 0; c < copies; ++c)
+      check(hipMemcpyAsync(stage + c * m, src + c * n + begin, values * sizeof(float), hipMemcpyDeviceToHost, ctx.stream()), what);
+    ctx.sync();
+    double* to = out + C * begin;
+    parallel_for(m, [=](size_t b, size_t e) {
+      for (size_t i = b; i < e; ++i)
+        for (size_t c = 0; c < C; ++c) to[C * i + c] = double(stage[c * m + i]);
+    });
+  }
+}
+
 void HipBackend::download_image_to(const HImage& im, double* out) {
-  const size_t n = im.grid.num_voxels();
-  auto* stage = static_cast<float*>(ctx_->pinned(n * sizeof(float)));
-  check(hipMemcpyAsync(stage, im.buf.get(), n * sizeof(float), hipMemcpyDeviceToHost, ctx_->stream()), "download image");
-  ctx_->sync();
-  parallel_for(n, [&](size_t b, size_t e) {
-    for (size_t i = b; i < e; ++i) out[i] = double(stage[i]);
-  });
+  download_planes<1>(*ctx_, im.buf.get(), im.grid.num_voxels(), out, "download image");
 }
 
 HField HipBackend::zero_field(const Grid& g) {
@@ -458,17 +475,7 @@ HField HipBackend::upload_field(const VectorField& v) {
 
 void HipBackend::download_field_to(const HField& f, double* aos) {
   HostTimer host_timer("download_field");
-  const size_t n = f.grid.num_voxels();
-  auto* stage = static_cast<float*>(ctx_->pinned(3 * n * sizeof(float)));
-  check(hipMemcpyAsync(stage, f.buf.get(), 3 * n * sizeof(float), hipMemcpyDeviceToHost, ctx_->stream()), "download field");
-  ctx_->sync();
-  parallel_for(n, [&](size_t b, size_t e) {
-    for (size_t i = b; i < e; ++i) {
-      aos[3 * i] = double(stage[i]);
-      aos[3 * i + 1] = double(stage[n + i]);
-      aos[3 * i + 2] = double(stage[2 * n + i]);
-    }
-  });
+  download_planes<3>(*ctx_, f.buf.get(), f.grid.num_voxels(), aos, "download field");
 }
 
 VectorField HipBackend::download_field(const HField& f) {
