@@ -219,10 +219,8 @@ const TuningTable& default_tuning();
 
 // The planes a CC block walks on grid d under tuning table t (knobs cc.tile_z, cc.min_blocks; the
 // split that takes the least time where neither is set).
-// The kernel addresses a tile's rows with 32-bit byte offsets from the first.
+static_assert(4ull * Grid::kMaxAxis * (kCcTileY + 2 * 8) < (1ull << 32), "a CC tile's rows are addressed with 32-bit byte offsets");
 inline int cc_tile(const TuningTable& t, const Dims& d, int radius) {
-  if (4ll * d.nx * std::min(kCcTileY + 2 * radius, d.ny) >= (1ll << 32))
-    invalid("hip backend", "cc: rows of " + std::to_string(d.nx) + " voxels are not supported");
   const uint64_t n = uint64_t(d.n());
   const int tile = int(t.get("cc.tile_z", n, 0)), blocks = int(t.get("cc.min_blocks", n, 0));
   if (tile == 0 && blocks == 0) return cc_tile_for(d, radius, 0, 0);

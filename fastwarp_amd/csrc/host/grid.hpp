@@ -16,6 +16,8 @@ struct Grid {
   Mat3 direction = kIdentity3;  // axis directions as columns: direction[row][axis]
   Mat3 index_from_offset = kIdentity3;
 
+  static constexpr size_t kMaxAxis = size_t(1) << 20;
+
   Grid() = default;
 
   // grid.rs:46-88 `Grid::new`: rejects zero sizes, overflowing voxel counts, non-positive or
@@ -23,7 +25,7 @@ struct Grid {
   Grid(std::array<size_t, 3> sz, Vec3 sp, Vec3 org, Mat3 dir) : size(sz), spacing(sp), origin(org), direction(dir) {
     for (size_t s : size)
       if (s == 0) invalid("grid", "zero size");
-    if (size[0] > (size_t(1) << 20) || size[1] > (size_t(1) << 20) || size[2] > (size_t(1) << 20))
+    if (size[0] > kMaxAxis || size[1] > kMaxAxis || size[2] > kMaxAxis)
       invalid("grid", "voxel count overflows");
     for (double s : spacing)
       if (!std::isfinite(s) || s <= 0.0) invalid("grid", "spacing must be positive and finite");
