@@ -223,8 +223,8 @@ static_assert(4ull * Grid::kMaxAxis * (kCcTileY + 2 * 8) < (1ull << 32), "a CC t
 inline int cc_tile(const TuningTable& t, const Dims& d, int radius) {
   const uint64_t n = uint64_t(d.n());
   const int tile = int(t.get("cc.tile_z", n, 0)), blocks = int(t.get("cc.min_blocks", n, 0));
-  if (tile == 0 && blocks == 0) return cc_tile_for(d, radius, 0, 0);
-  return cc_tile_for(d, radius, tile ? tile : kCcTileZ, blocks ? blocks : kCcMinBlocks);
+  if (tile == 0 && blocks == 0) return cc_run(d.nx, d.ny, d.nz, radius, 0, 0);
+  return cc_run(d.nx, d.ny, d.nz, radius, tile ? tile : kCcTileZ, blocks ? blocks : kCcMinBlocks);
 }
 
 // A scalar image on the device (f32, x-fastest).

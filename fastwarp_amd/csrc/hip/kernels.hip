@@ -49,7 +49,7 @@ LaunchEvents*& current_launch_events() {
 // sums of split values, running along z with the leaving plane subtracted, on 64 x 8 tiles: 375 us
 // (radius 2: 120 for 305, radius 8: 329 for 952; 45 x 54 x 45 at radius 4: 22 for 51).
 // ------------------------------------------------------------------------------------------
-constexpr int kCcTX = 32, kCcTY = kCcTileY, kCcThreads = kCcTX * kCcTY;
+constexpr int kCcTX = kCcTileX, kCcTY = kCcTileY, kCcThreads = kCcTX * kCcTY;
 constexpr int kCcRun = 8;  // outputs along x of one lane of the x pass
 
 template <int R>
@@ -261,35 +261,6 @@ void launch_cc_items(const CcItems& c, hipStream_t s) {
 
 dim3 cc_grid(const Dims& d, int tile_z) {
   return dim3((d.nx + kCcTX - 1) / kCcTX, (d.ny + kCcTY - 1) / kCcTY, (d.nz + tile_z - 1) / tile_z);
-}
-
-// The z run of a CC block. With a choice of the tuning table: the longest of max_tile, max_tile / 2,
-// ..., 1 planes whose grid still has min_blocks blocks. By default (max_tile 0) the run that takes
-// the least time: a block walks tile_z + 2R planes one after another, a CU holds two blocks (187
-// registers at radius 4), and a plane takes a pair of blocks kCcPairTime times a block alone (both
-// are bound by f64 arithmetic for most of it).
-constexpr double kCcPairTime = 1.5;
-int cc_tile_for(const Dims& d, int radius, int max_tile, int min_blocks) {
-  const long long tiles = (long long)((d.nx + kCcTX - 1) / kCcTX) * ((d.ny + kCcTY - 1) / kCcTY);
-  if (max_tile > 0) {
-    int t = max_tile;
-    for (; t > 1; t /= 2)
-      if (tiles * ((d.nz + t - 1) / t) >= std::max(1, min_blocks)) break;
-    return t;
-  }
-  int best = d.nz;
-  double least = 1e300;
-  // at most kCcMostBlocks blocks, beyond one a tile
-  for (long long chunks = 1; chunks <= d.nz && (chunks == 1 || chunks * tiles <= kCcMostBlocks); ++chunks) {
-    const int t = (int)((d.nz + chunks - 1) / chunks);
-    const long long per_cu = (tiles * ((d.nz + t - 1) / t) + kCcCus - 1) / kCcCus;
-    const double time = double(t + 2 * radius) * (double(per_cu / 2) * kCcPairTime + double(per_cu % 2));
-    if (time < least) {
-      least = time;
-      best = t;
-    }
-  }
-  return best;
 }
 
 void launch_cc_pair(const CcArgs& a, hipStream_t s) {

@@ -8,6 +8,8 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
+#include "cc_split.hpp"
+
 namespace fw::hip {
 
 // Events carried by the launches of an open timing scope on this thread: the scope's first launch
@@ -69,12 +71,6 @@ struct CcArgs {
 };
 void launch_cc_pair(const CcArgs& a, hipStream_t s);
 dim3 cc_grid(const Dims& d, int tile_z);
-// The planes a CC block walks: by default (max_tile 0) the split that takes the least time, else the
-// longest run of at most max_tile planes (halving) whose grid still has min_blocks blocks.
-int cc_tile_for(const Dims& d, int radius, int max_tile, int min_blocks);
-constexpr int kCcTileZ = 16, kCcMinBlocks = 512;  // where the table sets only the other knob
-constexpr long long kCcCus = 256, kCcMostBlocks = 8192;
-constexpr int kCcTileY = 8;  // a CC block's rows
 
 // --- per-block partial reductions ---
 // Largest |u/spacing| of two fields (b may be null) and sums of squares.

@@ -29,13 +29,6 @@ void set_call_error(const std::string& message);
 namespace fw::hip {
 namespace {
 
-// The largest grid the entry point takes, in units of 64 x 8 x (at most 16) voxels (1 mm: 1,008).
-constexpr long long kNoAllocMaxUnits = 16384;
-// Every grid within that limit takes at most two CC blocks (32 x 8 voxels over a run of planes) a
-// unit: one for each half of a unit's columns where the run is at least the unit's, and by the
-// default rule at most kCcMostBlocks blocks where it is shorter.
-constexpr int kNoAllocMaxBlocks = 2 * int(kNoAllocMaxUnits);
-static_assert(kCcMostBlocks <= kNoAllocMaxBlocks, "the scratch holds every default z split");
 // Layout in 4-byte words: CC value partials (f32), CC counts (i32).
 constexpr size_t kOffCc = 0;
 constexpr size_t kOffCount = kOffCc + kNoAllocMaxBlocks;
@@ -43,18 +36,6 @@ constexpr size_t kScratchWords = kOffCount + kNoAllocMaxBlocks;
 
 // 262,144 bytes per device.
 static __device__ __align__(256) uint32_t scratch[kScratchWords];
-
-// The units of grid d: runs of 16 planes, halved while the grid has fewer than 512 units (grids of
-// 2^22 to 2^23 - 1 voxels: runs of 64, 256 units).
-long long noalloc_units(const Dims& d) {
-  const long long n = d.n();
-  const bool mid = n >= (1ll << 22) && n < (1ll << 23);
-  const long long columns = (long long)((d.nx + 63) / 64) * ((d.ny + 7) / 8);
-  for (int t = mid ? 64 : 16;; t /= 2) {
-    const long long units = columns * ((d.nz + t - 1) / t);
-    if (t == 1 || units >= (mid ? 256 : 512)) return units;
-  }
-}
 
 // values[0] = values[1] = -(sum of the block partials) / (sum of the counts), the block partials
 // added in block order in f64 as fw_cc_pair adds them on the host: 256 threads stage them in LDS
@@ -135,10 +116,15 @@ extern "C" int fw_cc_pair_noalloc(const fw_grid* grid, const float* fixed, const
     a.tile_z = cc_tile(default_tuning(), a.d, a.radius);
     const dim3 gr = cc_grid(a.d, a.tile_z);
     const long long blocks = (long long)gr.x * gr.y * gr.z;
-    const long long units = noalloc_units(a.d);
-    if (units > kNoAllocMaxUnits || blocks > kNoAllocMaxBlocks)
-      fw::invalid("cc noalloc", "the grid has " + std::to_string(units) + " units of 64 x 8 x 16 voxels, more than the " +
-                                    std::to_string(kNoAllocMaxUnits) + " the static scratch holds");
+    const uint64_t n = uint64_t(a.d.n());
+    const long long units = noalloc_units(a.d.nx, a.d.ny, a.d.nz, int(default_tuning().get("cc.tile_z", n, 0)),
+                                          int(default_tuning().get("cc.min_blocks", n, 0)));
+    if (units > kNoAllocMaxUnits)
+      fw::invalid("cc noalloc", "the grid has " + std::to_string(units) + " units of 64 x 8 columns over a z run, more than the " +
+                                    std::to_string(kNoAllocMaxUnits) + " that a call with static scratch takes");
+    if (blocks > kNoAllocMaxBlocks)
+      fw::invalid("cc noalloc", "the grid needs " + std::to_string(blocks) + " CC blocks, more than the " +
+                                    std::to_string(kNoAllocMaxBlocks) + " the static scratch holds");
     uint32_t* ptr = scratch_of_current_device();
     a.probes = probes_of(g);
     a.d_fixed = d_fixed;

@@ -160,9 +160,9 @@ int fw_cc_pair(fw_ctx* ctx, const fw_image* fixed, const fw_image* moving, const
  * three planes each, written), values (2 f64, written: values[0] = values[1], as fw_cc_pair's).
  * The work is enqueued on `stream` (a hipStream_t, NULL for the null stream) and the call returns
  * without waiting; nothing is allocated. Block partials live in a static per-device scratch of
- * 262,144 bytes, which limits the grid to 16,384 units of 64 x 8 x (at most 16) voxels (the
- * 1 mm grid has 1008); a larger grid is rejected with FW_ERR_INVALID. Calls that overlap on one
- * GPU race on that scratch. Results are the same bits as fw_cc_pair's on the same images. Errors:
+ * 262,144 bytes. A grid of more than 16,384 units of 64 x 8 columns over a z run (16 planes, or the
+ * tuning table's cc.tile_z) is rejected with FW_ERR_INVALID: 1024 x 1024 x 128 voxels are the limit,
+ * the 1 mm grid has 504. Calls that overlap on one GPU race on that scratch. Results are the same bits as fw_cc_pair's on the same images. Errors:
  * the status, and fw_last_error(NULL) for the text. */
 int fw_cc_pair_noalloc(const fw_grid* grid, const float* fixed, const float* moving, uint32_t radius, float* d_fixed,
                        float* d_moving, double* values, void* stream);

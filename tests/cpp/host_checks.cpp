@@ -16,6 +16,7 @@
 
 #include <unistd.h>
 
+#include "../../fastwarp_amd/csrc/hip/cc_split.hpp"
 #include "../../fastwarp_amd/csrc/hip/fastdiv.hpp"
 #include "../../fastwarp_amd/csrc/host/admission.hpp"
 #include "../../fastwarp_amd/csrc/host/gauss_taps.hpp"
@@ -1062,8 +1063,37 @@ static void grow_buffer() {
   ok("grow_buffer");
 }
 
+// The CC entry point that cannot allocate: the limit it states, and that its scratch holds the blocks of
+// every grid within it, with the shipped table's choices and with a user's.
+static void noalloc_limits() {
+  using namespace fw::hip;
+  CHECK(noalloc_units(182, 218, 182, 0, 0) == 504 && noalloc_units(1024, 1024, 128, 0, 0) == 16384, "the stated units");
+  CHECK(noalloc_units(1024, 1024, 512, 0, 0) == 65536, "a grid beyond the limit");
+  // a table with longer runs takes deeper grids, one with shorter runs fewer
+  CHECK(noalloc_units(1024, 1024, 512, 64, 1) == 16384, "runs of 64 planes");
+  CHECK(noalloc_units(1024, 1024, 32, 1, 0) == 65536, "runs of one plane");
+  const int sizes[] = {1, 3, 8, 31, 33, 63, 64, 65, 100, 182, 256, 511, 1024, 4096, 1 << 20};
+  long long taken = 0;
+  for (int nx : sizes)
+    for (int ny : sizes)
+      for (int nz : sizes)
+        for (int tile : {0, 1, 5, 16, 64, 256})
+          for (int blocks : {0, 1, 256, 65536}) {
+            if (noalloc_units(nx, ny, nz, tile, blocks) > kNoAllocMaxUnits) continue;
+            ++taken;
+            for (int radius = 1; radius <= 8; ++radius) {
+              const int t = tile == 0 && blocks == 0 ? cc_run(nx, ny, nz, radius, 0, 0)
+                                                     : cc_run(nx, ny, nz, radius, tile ? tile : kCcTileZ, blocks ? blocks : kCcMinBlocks);
+              CHECK(t >= 1 && cc_columns(nx, ny) * ((nz + t - 1) / t) <= kNoAllocMaxBlocks, "the scratch holds the blocks");
+            }
+          }
+  CHECK(taken > 10000, "grids within the limit");
+  ok("noalloc_limits");
+}
+
 int main() {
   grow_buffer();
+  noalloc_limits();
   host_loops();
   mt19937();
   regular_sampling();
