@@ -1,7 +1,7 @@
 """Builds the gfx950 shared library `fastwarp_amd/lib/libfastwarp_hip.so` in-tree with hipcc.
 
-Every translation unit is compiled in parallel into `fastwarp_amd/_build/`, then linked. HIP code
-is compiled with the packed-FP32 instructions disabled (`-packed-fp32-ops`).
+Every translation unit is compiled in parallel into `fastwarp_amd/_build/`, then linked (the CC
+kernels as one object per window radius). HIP code is compiled with the packed-FP32 instructions disabled (`-packed-fp32-ops`).
 """
 from __future__ import annotations
 
@@ -56,20 +56,20 @@ def _run(cmds: list[list[str]]) -> None:
         raise RuntimeError(f"{len(failed)} compile step(s) failed")
 
 
+def objects() -> list[tuple[Path, Path, list[str]]]:
+    """(source, object, further flags) of every compile step, the longest ones first."""
+    cc = CSRC / "hip" / "cc.hip"
+    steps = [(cc, BUILD / f"cc_r{r}.o", [f"-DFW_CC_RADIUS={r}"]) for r in range(8, 0, -1)]
+    return steps + [(src, BUILD / (src.name + ".o"), []) for src in SOURCES]
+
+
 def build(verbose: bool = False) -> Path:
     BUILD.mkdir(exist_ok=True)
     LIB.parent.mkdir(exist_ok=True)
-    objs = []
-    cmds = []
-    for src in SOURCES:
-        if not src.exists():
-            continue
-        obj = BUILD / (src.name + ".o")
-        objs.append(obj)
-        cmds.append([HIPCC, *FLAGS, "-c", str(src), "-o", str(obj)])
-    _run(cmds)
+    steps = objects()
+    _run([[HIPCC, *FLAGS, *extra, "-c", str(src), "-o", str(obj)] for src, obj, extra in steps])
     tmp = LIB.with_suffix(".so.tmp")
-    _run([[HIPCC, *FLAGS, "-shared", *map(str, objs), "-o", str(tmp), "-lpthread"]])
+    _run([[HIPCC, *FLAGS, "-shared", *[str(obj) for _, obj, _ in steps], "-o", str(tmp), "-lpthread"]])
     os.replace(tmp, LIB)
     if verbose:
         print(f"built {LIB}")

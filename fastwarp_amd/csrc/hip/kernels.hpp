@@ -70,6 +70,9 @@ struct CcArgs {
   int* partial_count;    // per block: valid voxels
 };
 void launch_cc_pair(const CcArgs& a, hipStream_t s);
+// The launch of one radius (1 to 8).
+template <int R>
+void launch_cc_radius(const CcArgs& a, hipStream_t s);
 dim3 cc_grid(const Dims& d, int tile_z);
 
 // --- per-block partial reductions ---
@@ -220,6 +223,8 @@ struct CcItems {
   int count;
 };
 void launch_cc_items(const CcItems& c, hipStream_t s);
+template <int R>
+void launch_cc_items_radius(const CcItems& c, hipStream_t s);
 struct NormItems {
   const float* a[kBatchItems];
   const float* b[kBatchItems];
