@@ -594,8 +594,10 @@ MetricPair<HField> HipBackend::cc_pair(const HImage& fixed, const HImage& moving
   a.valid = valid ? valid->buf.get() : nullptr;
   a.d = dims_of(g);
   a.radius = int(radius);
-  a.tile_z = cc_tile(ctx_->tuning(), a.d, a.radius);
   a.probes = probes_of(g);
+  const CcPlan plan = cc_plan(ctx_->tuning(), a.d, a.radius, a.valid != nullptr, a.probes);
+  a.tile_z = plan.run;
+  a.plane = plan.plane;
   a.d_fixed = out.fields[0].buf.get();
   a.d_moving = out.fields[1].buf.get();
   const dim3 gr = cc_grid(a.d, a.tile_z);
@@ -630,12 +632,7 @@ MetricPair<HField> HipBackend::cc_pair(const HImage& fixed, const HImage& moving
   ctx_->sync();
   const float* pcc = reinterpret_cast<const float*>(host);
   const int* pcount = reinterpret_cast<const int*>(host + real * sizeof(float));
-  double total = 0.0;
-  long long count = 0;
-  for (size_t b = 0; b < real; ++b) {
-    total += double(pcc[b]);
-    count += pcount[b];
-  }
+  const auto [total, count] = cc_total(pcc, pcount, real);
   if (count == 0)
     invalid("cc metric", valid ? "no voxel of the registration level lies inside both the fixed and the moving mask"
                                : "no virtual voxel maps inside both image buffers");
@@ -669,8 +666,10 @@ MetricPair<HField> HipBackend::cc_pair_deferred(const HImage& fixed, const HImag
   a.valid = nullptr;
   a.d = dims_of(g);
   a.radius = int(radius);
-  a.tile_z = cc_tile(ctx_->tuning(), a.d, a.radius);
   a.probes = probes_of(g);
+  const CcPlan plan = cc_plan(ctx_->tuning(), a.d, a.radius, a.valid != nullptr, a.probes);
+  a.tile_z = plan.run;
+  a.plane = plan.plane;
   a.d_fixed = out.fields[0].buf.get();
   a.d_moving = out.fields[1].buf.get();
   const dim3 gr = cc_grid(a.d, a.tile_z);
@@ -708,12 +707,7 @@ MetricPair<HField> HipBackend::cc_pair_deferred(const HImage& fixed, const HImag
   out.later = Pending<std::array<double, 2>>(std::function<std::array<double, 2>()>([host, real] {
     const float* pcc = reinterpret_cast<const float*>(host);
     const int* pcount = reinterpret_cast<const int*>(host + real * sizeof(float));
-    double total = 0.0;
-    long long count = 0;
-    for (size_t b = 0; b < real; ++b) {
-      total += double(pcc[b]);
-      count += pcount[b];
-    }
+    const auto [total, count] = cc_total(pcc, pcount, real);
     if (count == 0) invalid("cc metric", "no virtual voxel maps inside both image buffers");
     const double v = -total / double(count);
     return std::array<double, 2>{v, v};

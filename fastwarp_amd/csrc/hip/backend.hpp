@@ -217,14 +217,12 @@ class DevBuf {
 // tuning/gfx950.json beside the library's directory (fastwarp_amd/tuning/ for lib/), else empty.
 const TuningTable& default_tuning();
 
-// The planes a CC block walks on grid d under tuning table t (knobs cc.tile_z, cc.min_blocks; the
-// split that takes the least time where neither is set).
+// The CC launch of grid d under tuning table t (knobs cc.tile_z, cc.min_blocks).
 static_assert(4ull * Grid::kMaxAxis * (kCcTileY + 2 * 8) < (1ull << 32), "a CC tile's rows are addressed with 32-bit byte offsets");
-inline int cc_tile(const TuningTable& t, const Dims& d, int radius) {
+inline CcPlan cc_plan(const TuningTable& t, const Dims& d, int radius, bool masked, const Probes& probes) {
   const uint64_t n = uint64_t(d.n());
-  const int tile = int(t.get("cc.tile_z", n, 0)), blocks = int(t.get("cc.min_blocks", n, 0));
-  if (tile == 0 && blocks == 0) return cc_run(d.nx, d.ny, d.nz, radius, 0, 0);
-  return cc_run(d.nx, d.ny, d.nz, radius, tile ? tile : kCcTileZ, blocks ? blocks : kCcMinBlocks);
+  return cc_plan(d.nx, d.ny, d.nz, radius, masked, probes.diagonal != 0, int(t.get("cc.tile_z", n, 0)),
+                 int(t.get("cc.min_blocks", n, 0)));
 }
 
 // A scalar image on the device (f32, x-fastest).

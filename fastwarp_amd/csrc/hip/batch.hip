@@ -191,7 +191,8 @@ struct LevelBuffers {
   std::vector<HField> smoothed;                 // [2k]
   std::vector<DevBuf> tmp;                      // [2k] the x/y pass of the two-pass smoothing
   DevBuf norm_parts, coef, step_parts, factors;
-  int nb = 0, tile_z = 0;
+  int nb = 0;
+  CcPlan cc{};
   size_t blocks = 0;
   char* cc_host = nullptr;
   float* pcc_dev = nullptr;
@@ -245,8 +246,8 @@ std::unique_ptr<LevelBuffers> make_level_buffers(HipBackend& b, const SynRecipe&
   }
   L->step_parts = DevBuf(&ctx, k * 4 * size_t(L->nb));
   L->factors = DevBuf(&ctx, 2 * k);
-  L->tile_z = cc_tile(ctx.tuning(), d, int(recipe.cc_radius));
-  const dim3 gr = cc_grid(d, L->tile_z);
+  L->cc = cc_plan(ctx.tuning(), d, int(recipe.cc_radius), false, probes_of(g));
+  const dim3 gr = cc_grid(d, L->cc.run);
   L->blocks = size_t(gr.x) * gr.y * gr.z;
   // coherent host memory for the whole level (later, smaller active sets fit in it)
   void* cc_dev = nullptr;
@@ -369,7 +370,8 @@ void issue_updates(HipBackend& b, const SynRecipe& recipe, const std::vector<dou
       a.valid = nullptr;
       a.d = d;
       a.radius = int(recipe.cc_radius);
-      a.tile_z = L.tile_z;
+      a.tile_z = L.cc.run;
+      a.plane = L.cc.plane;
       a.probes = probes_of(g);
       a.d_fixed = L.dfix[q][c].buf.get();
       a.d_moving = L.dmov[q][c].buf.get();
@@ -578,18 +580,14 @@ void iterate(HipBackend& b, const SynRecipe& recipe, const std::vector<double>& 
         invalid("syn", "the displacement field is not finite");
     }
     if (nc > 1 && bad_host[q]) invalid("syn", "the metric gradient is not finite");
-    // the channels' values, each from its block partials in block order
+    // the channels' values, each from its block partials
     const float* pcc = reinterpret_cast<const float*>(L.cc_host);
     const int* pcount = reinterpret_cast<const int*>(L.cc_host + L.k * nc * L.blocks * sizeof(float));
     double weighted[2] = {0.0, 0.0};
     double first = 0.0;
     for (size_t c = 0; c < nc; ++c) {
-      double total = 0.0;
-      long long count = 0;
-      for (size_t bl = 0; bl < L.blocks; ++bl) {
-        total += double(pcc[(q * nc + c) * L.blocks + bl]);
-        count += pcount[(q * nc + c) * L.blocks + bl];
-      }
+      const size_t at = (q * nc + c) * L.blocks;
+      const auto [total, count] = cc_total(pcc + at, pcount + at, L.blocks);
       if (count == 0) invalid("cc metric", "no virtual voxel maps inside both image buffers");
       const double v = -total / double(count);
       if (c == 0) first = v;

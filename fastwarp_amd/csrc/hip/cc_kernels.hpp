@@ -33,9 +33,9 @@ namespace fw::hip {
 // running window from partial sums (three or four additions a plane, CcWindow).
 //
 // Bound by the latency of its f64 chains at two waves a SIMD (vector instructions fill a third of the
-// time, the LDS reads of the y pass another). 182 x 218 x 182, radius 4, with the value's sum: 156 us;
-// sums of split values, running along z with the leaving plane subtracted, on 64 x 8 tiles: 375 us
-// (radius 2: 120 for 305, radius 8: 329 for 952; 45 x 54 x 45 at radius 4: 22 for 51).
+// time, the LDS reads of the y pass another). 182 x 218 x 182, radius 4, inputs in cache: 147 us; sums of
+// split values, running along z with the leaving plane subtracted, on 64 x 8 tiles: 337 us (radius 2: 118
+// for 262, radius 8: 323 for 947). With the value's sum and inputs from HBM: 177 us for 391.
 // ------------------------------------------------------------------------------------------
 constexpr int kCcTX = kCcTileX, kCcTY = kCcTileY, kCcThreads = kCcTX * kCcTY;
 constexpr int kCcRun = 8;  // outputs along x of one lane of the x pass
@@ -170,6 +170,46 @@ __device__ __forceinline__ double mean_of(double sum, double count, double inv_c
   return fma(fma(-q, count, sum), inv_count, q);
 }
 
+// A window's means, centred moments and local CC from its five sums (cc.rs:270-300), and the
+// coefficients of the two derivative directions at its centre values.
+struct CcPoint {
+  double fmean, mmean, s_ff, s_mm, s_fm, r, cc;
+  __device__ __forceinline__ CcPoint(const double (&w)[5], double count, double inv_count)
+      : fmean(mean_of(w[0], count, inv_count)), mmean(mean_of(w[1], count, inv_count)) {
+    s_ff = fma(-fmean, w[0], w[2]);
+    s_mm = fma(-mmean, w[1], w[3]);
+    s_fm = fma(-fmean, w[1], w[4]);
+    const double product = s_ff * s_mm;
+    r = reciprocal(product);
+    cc = fabs(product) > (double)kEps64 ? s_fm * s_fm * r : 1.0;
+  }
+  __device__ __forceinline__ bool varies() const { return s_ff > (double)kEps64 && s_mm > (double)kEps64; }
+  // 2 s_fm / (s_ff s_mm) and the regression slopes s_fm / s_mm, s_fm / s_ff from one reciprocal
+  __device__ __forceinline__ void coefficients(double fc, double mc, double& cf, double& cm) const {
+    const double fi = fc - fmean, mi = mc - mmean;
+    const double k1 = s_fm * r;
+    cf = 2.0 * k1 * fma(-k1 * s_ff, mi, fi);
+    cm = 2.0 * k1 * fma(-k1 * s_mm, fi, mi);
+  }
+};
+
+// Along grid axis g of an axis-aligned grid: the factor of the difference of the two neighbours, and the
+// plane (physical axis) its product goes to.
+struct CcAxes {
+  float fac[3] = {0.0f, 0.0f, 0.0f};
+  int plane[3] = {0, 1, 2};
+  __device__ __forceinline__ explicit CcAxes(const Probes& pr) {
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+#pragma unroll
+      for (int g = 0; g < 3; ++g)
+        if (pr.o[p][g] != 0.0f) {
+          fac[g] = (pr.o[p][g] > 0.0f ? 0.5f : -0.5f) * pr.inv_spacing[p];
+          plane[g] = p;
+        }
+  }
+};
+
 static __device__ float block_sum_f64(double v) {
   __shared__ double red[16];
   for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
@@ -184,7 +224,9 @@ static __device__ float block_sum_f64(double v) {
 }
 
 // Waves per SIMD the registers are held to. At radius 4 the windows take 80 registers and the kernel
-// 187: held to 168 for three blocks a CU it spills 21 of them and takes 199 us at 1 mm for 156 us.
+// 187: held to 168 for three blocks a CU it spills 21 of them and takes 199 us at 1 mm for 156 us. Up to
+// radius 3 an axis-aligned grid's kernel fits 168 (110 to 165). From radius 7 on (6 with a mask, 4 oblique with
+// one) the windows exceed the 256 of two waves and 4 to 120 registers are spilled.
 template <int R>
 constexpr int cc_waves() {
   return R <= 3 ? 3 : 2;
@@ -211,25 +253,216 @@ __global__ __launch_bounds__(kCcThreads, cc_waves<R>()) void k_cc2_items(CcItems
 #undef FW_CC2_TILE
 }
 
-template <int R, bool M>
-static void launch_cc_r(const CcArgs& a, hipStream_t s) {
-  if (a.probes.diagonal) launch((k_cc2<R, M, true>), cc_grid(a.d, a.tile_z), dim3(kCcThreads), 0, s, a);
-  else launch((k_cc2<R, M, false>), cc_grid(a.d, a.tile_z), dim3(kCcThreads), 0, s, a);
+// ------------------------------------------------------------------------------------------
+// The same pair one plane at a time, where the grid gives too few blocks for long walks (cc_plan). Each
+// thread sums its columns of the tile and halo over the window's planes first, with all loads independent
+// of each other, then the x and y passes run once, in place, where k_cc2 runs them for every plane of the
+// window. The sums are the same terms in f64 in another order, none subtracted.
+//
+// Bound by the z pass (2R + 1 planes of 2.5 columns a thread at radius 4, from L2) where the chip is full
+// and by one chain of loads, three barriers and the f64 sums where it is not: at radius 4 7.9 us at
+// 24 x 28 x 24 (k_cc2 15.8), 11.6 at 45 x 54 x 45 (19).
+// ------------------------------------------------------------------------------------------
+template <int R, bool MASKED, bool DIAGONAL>
+__device__ __forceinline__ void cc_plane(const CcArgs& a, uint3 bl) {
+  using T = CcTile<R>;
+  constexpr int W = T::W, SUMS = MASKED ? 6 : 5;
+  // odd, so that the x pass's eight rows a half-wave lie on different banks
+  constexpr int PITCH = T::LX | 1;
+  constexpr int ROWS = SUMS * T::LY * T::RUNS, JOBS = (ROWS + kCcThreads - 1) / kCcThreads;
+  __shared__ double sums[SUMS][T::LY * PITCH];
+  const Dims d = a.d;
+  const int x0 = bl.x * kCcTX, y0 = bl.y * kCcTY, z0 = bl.z * a.tile_z, z1 = min(z0 + a.tile_z, d.nz);
+  const long long plane = (long long)d.nx * d.ny, n3 = d.n();
+
+  const CcAxes axes(a.probes);
+  double cc_sum = 0.0;
+  int counted = 0;
+#pragma unroll 1
+  for (int z = z0; z < z1; ++z) {
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // offsets are formed for each plane: hoisted, they take the registers of two waves
+    // z pass
+#pragma unroll
+    for (int q = 0; q < T::PER; ++q) {
+      const int e = tid + kCcThreads * q;
+      const int ly = e / T::LX, lx = e % T::LX;
+      const int gx = x0 - R + lx, gy = y0 - R + ly;
+      const int cx = min(max(gx, 0), d.nx - 1), cy = min(max(gy, 0), d.ny - 1);
+      const long long o = (long long)cx + (long long)d.nx * cy;
+      double s[SUMS] = {};
+#pragma unroll
+      for (int t = 0; t < W; ++t) {
+        const int k = z - R + t;
+        const long long at = o + plane * min(max(k, 0), d.nz - 1);
+        float u = a.fixed[at], v = a.moving[at];
+        bool in = k >= 0 && k < d.nz;
+        if constexpr (MASKED) in = in && a.valid[at] != 0.0f;
+        u = in ? u : 0.0f;
+        v = in ? v : 0.0f;
+        s[0] += (double)u;
+        s[1] += (double)v;
+        s[2] = fma((double)u, (double)u, s[2]);
+        s[3] = fma((double)v, (double)v, s[3]);
+        s[4] = fma((double)u, (double)v, s[4]);
+        if constexpr (MASKED) s[5] += in ? 1.0 : 0.0;
+      }
+      if (T::LX * T::LY % kCcThreads == 0 || e < T::LX * T::LY) {
+        const bool in = gx == cx && gy == cy;
+#pragma unroll
+        for (int c = 0; c < SUMS; ++c) sums[c][ly * PITCH + lx] = in ? s[c] : 0.0;
+      }
+    }
+    __syncthreads();
+    // x pass: runs of kCcRun outputs of one row of one sum, written over the row once all are read
+    double o[JOBS][kCcRun];
+#pragma unroll
+    for (int q = 0; q < JOBS; ++q) {
+      const int e = min(tid + kCcThreads * q, ROWS - 1);
+      const double* row = &sums[0][0] + (e / T::RUNS) * PITCH + (e % T::RUNS) * kCcRun;
+      window_sums<kCcRun, W>([&](int t) { return row[t]; }, [&](int t, double v) { return v + row[t]; }, o[q]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < JOBS; ++q) {
+      const int e = tid + kCcThreads * q;
+      if (e < ROWS) {
+        double* row = &sums[0][0] + (e / T::RUNS) * PITCH + (e % T::RUNS) * kCcRun;
+#pragma unroll
+        for (int t = 0; t < kCcRun; ++t) row[t] = o[q][t];
+      }
+    }
+    __syncthreads();
+    // y pass and output
+    const int tx = tid & (kCcTX - 1), ty = tid / kCcTX;
+    const int x = x0 + tx, y = y0 + ty;
+    if (x < d.nx && y < d.ny) {
+      const long long at = lin(d, x, y, z);
+      float df[3] = {0.0f, 0.0f, 0.0f}, dm[3] = {0.0f, 0.0f, 0.0f};
+      if (!MASKED || a.valid[at] != 0.0f) {
+        double w[SUMS];
+#pragma unroll
+        for (int q = 0; q < SUMS; ++q) {
+          double s = 0.0;
+#pragma unroll
+          for (int t = 0; t < W; ++t) s += sums[q][(ty + t) * PITCH + tx];
+          w[q] = s;
+        }
+        double count;
+        if constexpr (MASKED) count = w[5];
+        else count = (double)(window_count(x, d.nx, R) * window_count(y, d.ny, R) * window_count(z, d.nz, R));
+        const double five[5] = {w[0], w[1], w[2], w[3], w[4]};
+        const CcPoint p(five, count, 1.0 / count);
+        cc_sum += p.cc;
+        counted += 1;
+        if (p.varies()) {
+          float gm[3], gf[3];
+          if constexpr (DIAGONAL) {
+            // the two neighbours along each grid axis, at the edges as k_cc2 reads them
+            const long long step[3] = {1, d.nx, plane};
+            const int pos[3] = {x, y, z}, len[3] = {d.nx, d.ny, d.nz};
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+              const long long up = pos[q] + 1 < len[q] ? step[q] : 0, down = pos[q] >= 1 && pos[q] + 1 < len[q] ? step[q] : 0;
+              gm[q] = (a.moving[at + up] - a.moving[at - down]) * axes.fac[q];
+              gf[q] = (a.fixed[at + up] - a.fixed[at - down]) * axes.fac[q];
+            }
+          } else {
+#pragma unroll 1
+            for (int q = 0; q < 3; ++q) {
+              gm[q] = central_difference(a.moving, d, a.probes, q, x, y, z);
+              gf[q] = central_difference(a.fixed, d, a.probes, q, x, y, z);
+            }
+          }
+          double cf, cm;
+          p.coefficients((double)a.fixed[at], (double)a.moving[at], cf, cm);
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            df[q] = (float)(cf * (double)gm[q]);
+            dm[q] = (float)(cm * (double)gf[q]);
+          }
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        const long long to = at + n3 * (DIAGONAL ? axes.plane[q] : q);
+        a.d_fixed[to] = df[q];
+        a.d_moving[to] = dm[q];
+      }
+    }
+    __syncthreads();  // the y pass has read the plane's sums
+  }
+  const float total = block_sum_f64(cc_sum);
+  const float cnt = block_sum((float)counted);
+  if (threadIdx.x == 0) {
+    const unsigned b = bl.x + gridDim.x * (bl.y + gridDim.y * bl.z);
+    a.partial_cc[b] = total;
+    a.partial_count[b] = (int)cnt;
+  }
+}
+
+template <int R, bool MASKED, bool DIAGONAL>
+__global__ __launch_bounds__(kCcThreads) void k_cc2_plane(CcArgs a) {
+  cc_plane<R, MASKED, DIAGONAL>(a, xcd_block());
+}
+
+template <int R, bool DIAGONAL>
+__global__ __launch_bounds__(kCcThreads) void k_cc2_plane_items(CcItems c) {
+  const unsigned gz = gridDim.z / (unsigned)c.count;
+  const uint3 bl = xcd_block();
+  const unsigned q = bl.z / gz;
+  cc_plane<R, false, DIAGONAL>(c.a[q], make_uint3(bl.x, bl.y, bl.z - q * gz));
+}
+
+// Whether k_cc2 is there for a radius: on oblique grids, whose gradient gathers leave it too few
+// registers, only where it is the faster one on large grids (cc_plan).
+template <int R, bool M, bool DIAGONAL>
+constexpr bool cc_walks() {
+  return DIAGONAL || R >= (M ? kCcObliqueMasked : kCcObliquePlain);
+}
+
+template <int R, bool M, bool DIAGONAL>
+static void launch_cc_one(const CcArgs& a, hipStream_t s) {
+  const dim3 g = cc_grid(a.d, a.tile_z), t(kCcThreads);
+  if constexpr (cc_walks<R, M, DIAGONAL>()) {
+    if (!a.plane) {
+      launch((k_cc2<R, M, DIAGONAL>), g, t, 0, s, a);
+      return;
+    }
+  }
+  launch((k_cc2_plane<R, M, DIAGONAL>), g, t, 0, s, a);
 }
 
 template <int R>
 void launch_cc_radius(const CcArgs& a, hipStream_t s) {
-  if (a.valid != nullptr) launch_cc_r<R, true>(a, s);
-  else launch_cc_r<R, false>(a, s);
+  if (a.valid != nullptr) {
+    if (a.probes.diagonal) launch_cc_one<R, true, true>(a, s);
+    else launch_cc_one<R, true, false>(a, s);
+  } else {
+    if (a.probes.diagonal) launch_cc_one<R, false, true>(a, s);
+    else launch_cc_one<R, false, false>(a, s);
+  }
+}
+
+template <int R, bool DIAGONAL>
+static void launch_cc_items_one(const CcItems& c, hipStream_t s) {
+  const CcArgs& a = c.a[0];
+  const dim3 t(kCcThreads);
+  dim3 g = cc_grid(a.d, a.tile_z);
+  g.z *= (unsigned)c.count;
+  if constexpr (cc_walks<R, false, DIAGONAL>()) {
+    if (!a.plane) {
+      launch((k_cc2_items<R, DIAGONAL>), g, t, 0, s, c);
+      return;
+    }
+  }
+  launch((k_cc2_plane_items<R, DIAGONAL>), g, t, 0, s, c);
 }
 
 template <int R>
 void launch_cc_items_radius(const CcItems& c, hipStream_t s) {
-  const CcArgs& a = c.a[0];
-  dim3 g = cc_grid(a.d, a.tile_z);
-  g.z *= (unsigned)c.count;
-  if (a.probes.diagonal) launch((k_cc2_items<R, true>), g, dim3(kCcThreads), 0, s, c);
-  else launch((k_cc2_items<R, false>), g, dim3(kCcThreads), 0, s, c);
+  if (c.a[0].probes.diagonal) launch_cc_items_one<R, true>(c, s);
+  else launch_cc_items_one<R, false>(c, s);
 }
 
 }  // namespace fw::hip

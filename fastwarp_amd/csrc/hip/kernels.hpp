@@ -62,7 +62,8 @@ struct CcArgs {
   const float* valid;  // nullptr: every voxel valid
   Dims d;
   int radius;
-  int tile_z;
+  int tile_z;  // planes of a block's run
+  bool plane;  // k_cc2_plane
   Probes probes;
   float* d_fixed;        // 3 planes: coefficient * grad(moving)
   float* d_moving;       // 3 planes: coefficient' * grad(fixed)

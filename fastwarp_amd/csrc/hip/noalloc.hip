@@ -37,34 +37,31 @@ constexpr size_t kScratchWords = kOffCount + kNoAllocMaxBlocks;
 // 262,144 bytes per device.
 static __device__ __align__(256) uint32_t scratch[kScratchWords];
 
-// values[0] = values[1] = -(sum of the block partials) / (sum of the counts), the block partials
-// added in block order in f64 as fw_cc_pair adds them on the host: 256 threads stage them in LDS
-// (one thread loading them from memory itself took 30 us for 1,008 blocks), one adds them.
-__global__ __launch_bounds__(256) void k_cc_value_final(const float* __restrict__ partial_cc, const int* __restrict__ count,
-                                                        int blocks, double* values) {
-  constexpr int kStage = 2048;
-  __shared__ float cc[kStage];
-  __shared__ int cn[kStage];
+// values[0] = values[1] = -(sum of the block partials) / (sum of the counts), the partials added in f64
+// in cc_total's order, as fw_cc_pair adds them on the host.
+__global__ __launch_bounds__(kCcLanes) void k_cc_value_final(const float* __restrict__ partial_cc, const int* __restrict__ count,
+                                                             int blocks, double* values) {
+  __shared__ double cc[kCcLanes];
+  __shared__ long long cn[kCcLanes];
+  const int t = threadIdx.x;
   double total = 0.0;
   long long c = 0;
-  for (int base = 0; base < blocks; base += kStage) {
-    const int m = min(kStage, blocks - base);
-    for (int b = threadIdx.x; b < m; b += blockDim.x) {
-      cc[b] = partial_cc[base + b];
-      cn[b] = count[base + b];
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-#pragma unroll 8
-      for (int b = 0; b < m; ++b) {
-        total += (double)cc[b];
-        c += cn[b];
-      }
-    }
-    __syncthreads();
+#pragma unroll 4
+  for (int b = t; b < blocks; b += kCcLanes) {
+    total += (double)partial_cc[b];
+    c += count[b];
   }
-  if (threadIdx.x != 0) return;
-  const double v = c > 0 ? -total / (double)c : __builtin_nan("");
+  cc[t] = total;
+  cn[t] = c;
+  for (int half = kCcLanes / 2; half > 0; half /= 2) {
+    __syncthreads();
+    if (t < half) {
+      cc[t] += cc[t + half];
+      cn[t] += cn[t + half];
+    }
+  }
+  if (t != 0) return;
+  const double v = cn[0] > 0 ? -cc[0] / (double)cn[0] : __builtin_nan("");
   values[0] = v;
   values[1] = v;
 }
@@ -112,8 +109,11 @@ extern "C" int fw_cc_pair_noalloc(const fw_grid* grid, const float* fixed, const
     a.valid = nullptr;
     a.d = dims_of(g);
     a.radius = int(radius);
-    // the same z runs as fw_cc_pair on a context with the default table, so the same bits
-    a.tile_z = cc_tile(default_tuning(), a.d, a.radius);
+    // the same launch as fw_cc_pair on a context with the default table, so the same bits
+    a.probes = probes_of(g);
+    const CcPlan plan = cc_plan(default_tuning(), a.d, a.radius, false, a.probes);
+    a.tile_z = plan.run;
+    a.plane = plan.plane;
     const dim3 gr = cc_grid(a.d, a.tile_z);
     const long long blocks = (long long)gr.x * gr.y * gr.z;
     const uint64_t n = uint64_t(a.d.n());
@@ -126,14 +126,13 @@ extern "C" int fw_cc_pair_noalloc(const fw_grid* grid, const float* fixed, const
       fw::invalid("cc noalloc", "the grid needs " + std::to_string(blocks) + " CC blocks, more than the " +
                                     std::to_string(kNoAllocMaxBlocks) + " the static scratch holds");
     uint32_t* ptr = scratch_of_current_device();
-    a.probes = probes_of(g);
     a.d_fixed = d_fixed;
     a.d_moving = d_moving;
     a.partial_cc = reinterpret_cast<float*>(ptr + kOffCc);
     a.partial_count = reinterpret_cast<int*>(ptr + kOffCount);
     hipStream_t s = static_cast<hipStream_t>(stream);
     launch_cc_pair(a, s);
-    launch(k_cc_value_final, dim3(1), dim3(256), 0, s, (const float*)a.partial_cc, (const int*)a.partial_count, int(blocks),
+    launch(k_cc_value_final, dim3(1), dim3(kCcLanes), 0, s, (const float*)a.partial_cc, (const int*)a.partial_count, int(blocks),
            values);
     if (hipGetLastError() != hipSuccess) throw std::runtime_error("fw_cc_pair_noalloc: kernel launch failed");
     return FW_OK;

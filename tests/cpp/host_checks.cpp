@@ -1082,18 +1082,39 @@ static void noalloc_limits() {
             if (noalloc_units(nx, ny, nz, tile, blocks) > kNoAllocMaxUnits) continue;
             ++taken;
             for (int radius = 1; radius <= 8; ++radius) {
-              const int t = tile == 0 && blocks == 0 ? cc_run(nx, ny, nz, radius, 0, 0)
-                                                     : cc_run(nx, ny, nz, radius, tile ? tile : kCcTileZ, blocks ? blocks : kCcMinBlocks);
-              CHECK(t >= 1 && cc_columns(nx, ny) * ((nz + t - 1) / t) <= kNoAllocMaxBlocks, "the scratch holds the blocks");
+              for (const bool diagonal : {false, true}) {
+                const int t = cc_plan(nx, ny, nz, radius, false, diagonal, tile, blocks).run;
+                CHECK(t >= 1 && cc_columns(nx, ny) * ((nz + t - 1) / t) <= kNoAllocMaxBlocks, "the scratch holds the blocks");
+              }
             }
           }
   CHECK(taken > 10000, "grids within the limit");
   ok("noalloc_limits");
 }
 
+// The CC launch: small grids one plane a block, large ones walked where the walking kernel is there, a table's
+// run as it says.
+static void cc_launches() {
+  using namespace fw::hip;
+  for (int radius = 1; radius <= 8; ++radius)
+    for (const bool masked : {false, true})
+      for (const bool diagonal : {false, true}) {
+        const bool walks = diagonal || radius >= (masked ? 4 : 7);
+        const CcPlan small = cc_plan(24, 28, 24, radius, masked, diagonal, 0, 0);
+        CHECK(small.plane && small.run == 1, "a small grid");
+        const CcPlan large = cc_plan(182, 218, 182, radius, masked, diagonal, 0, 0);
+        CHECK(large.plane == !walks && large.run > 1, "a large grid");
+        const CcPlan knob = cc_plan(24, 28, 24, radius, masked, diagonal, 5, 1);
+        CHECK(knob.plane == !walks && knob.run == 5, "a table's run");
+      }
+  CHECK(cc_plan(96, 112, 96, 4, false, true, 0, 0).plane && !cc_plan(96, 112, 97, 5, true, true, 0, 0).plane, "the lines");
+  ok("cc_launches");
+}
+
 int main() {
   grow_buffer();
   noalloc_limits();
+  cc_launches();
   host_loops();
   mt19937();
   regular_sampling();
