@@ -23,11 +23,19 @@ inline int halved_run(long long columns, int nz, int max_tile, int min_blocks) {
   return t;
 }
 
+// The time of `blocks` blocks of k_cc2 of one run on a CU, in units of a block alone. Its registers let two
+// run beside each other, three up to radius 3, four at radius 1; a second block adds 0.3, each further one
+// 0.25 (256 x 64 x 64 n grids in runs of 16 planes, launch taken off: 1 to 4 blocks a CU take 24, 31, 37, 43 us
+// at radius 1, 28, 36, 43, 64 at radius 2, 37, 49, 81, 94 at radius 4).
+inline double cc_cu_time(long long blocks, int radius) {
+  constexpr double beside[5] = {0.0, 1.0, 1.3, 1.55, 1.8};
+  const int fit = radius == 1 ? 4 : radius <= 3 ? 3 : 2;
+  return double(blocks / fit) * beside[fit] + beside[blocks % fit];
+}
+
 // The z run of a block of k_cc2 (which walks its planes one after another). With a choice of the tuning
 // table: halved_run of max_tile. By default (max_tile 0) the run that takes the least time: a block walks
-// tile_z + 2R planes, a CU holds two blocks (187 registers at radius 4), and a plane takes a pair of blocks
-// kCcPairTime times a block alone.
-constexpr double kCcPairTime = 1.5;
+// tile_z + 2R planes, and the fullest CU takes cc_cu_time.
 inline int cc_run(int nx, int ny, int nz, int radius, int max_tile, int min_blocks) {
   const long long tiles = cc_columns(nx, ny);
   if (max_tile > 0) return halved_run(tiles, nz, max_tile, min_blocks);
@@ -37,7 +45,7 @@ inline int cc_run(int nx, int ny, int nz, int radius, int max_tile, int min_bloc
   for (long long chunks = 1; chunks <= nz && (chunks == 1 || chunks * tiles <= kCcMostBlocks); ++chunks) {
     const int t = (int)((nz + chunks - 1) / chunks);
     const long long per_cu = (tiles * ((nz + t - 1) / t) + kCcCus - 1) / kCcCus;
-    const double time = double(t + 2 * radius) * (double(per_cu / 2) * kCcPairTime + double(per_cu % 2));
+    const double time = double(t + 2 * radius) * cc_cu_time(per_cu, radius);
     if (time < least) {
       least = time;
       best = t;
