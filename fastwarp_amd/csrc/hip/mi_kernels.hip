@@ -316,13 +316,8 @@ __global__ __launch_bounds__(1024) void k_mi_sampled_hist(MiSampledArgs a, HistM
   unsigned long long* mine = h + (k * COPIES + (COPIES == 1 ? 0 : (int)(threadIdx.x % COPIES))) * C;
   unsigned int valid = 0;
   const SampleRange rg = sample_range(a.count);
-  int s = rg.lo + ((int)threadIdx.x - k * group);
-  float4 next = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  if (s < rg.hi) next = a.samples[s];
-  while (s < rg.hi) {
-    const float4 smp = next;
-    s += group;
-    if (s < rg.hi) next = a.samples[s];  // in flight while this sample is binned
+  for (int s = rg.lo + ((int)threadIdx.x - k * group); s < rg.hi; s += group) {
+    const float4 smp = a.samples[s];
     const SampleEval e = eval_sample<WIDE>(a, map, smp);
     if (!e.ok) continue;
     ++valid;
