@@ -295,12 +295,15 @@ struct HistMaps<1> {
 
 // K transforms per pass over the same samples, each with its own histogram in the block's LDS (64-bit
 // atomics) and its own K-th of the block's threads, so that the transforms' gathers and atomics run
-// beside each other (one after another in every thread, a pass of four took 17.6 us on 3,267 samples
-// and 38 on 225,658, for 7.0 and 11.4 of one). A block writes its histograms to its own slot of
+// beside each other (one after another in every thread, a pass of four took 18.5 us on 3,267 samples
+// and 36.9 on 225,658; now 10.2 and 25.5). A block writes its histograms to its own slot of
 // `hist_slots`; a second kernel adds the slots, so the global histogram needs neither clearing nor
 // global atomics. With COPIES > 1 the lanes take turns over that many copies of the histogram, added
 // as the slot is written: most samples of a volume with background fall into a few cells, and the
 // additions of one wave to one cell are done one by one.
+//
+// Bound by the latency of one sample's gathers and atomics on small levels (3,267 samples: 6.5 us), by
+// the gathers on large ones (1.8 M: 20 us, 33.6 with one copy).
 template <int K, int COPIES, bool WIDE>
 __global__ __launch_bounds__(1024) void k_mi_sampled_hist(MiSampledArgs a, HistMaps<K> batch) {
   extern __shared__ unsigned long long h[];
@@ -349,9 +352,12 @@ int mi_batch_capacity(int bins) {
 // Images whose byte offsets do not fit 32 bits take the 64-bit form of the gathers.
 static bool wide_image(const MiSampledArgs& a) { return a.md.n() >= (1ll << 30); }
 
-// Blocks of at least this many samples keep copies of their histogram.
+// Copies of the histogram (1.8 M samples of a volume with background: 34.1 us with one, 21.3 with two, 20.0
+// with four, 20.3 with eight), kept by blocks of more than this many samples, whose threads then take
+// several one after another: 269 samples a block 7.6 us for 9.5, 440 10.3 for 11.8, 3,500 20 for 34. Below, each
+// thread has one sample (8.4 us either way on 101,000) and small levels would clear and add copies for nothing.
 constexpr int kMiCopies = 4;
-constexpr int kMiCopySamples = 2048;
+constexpr int kMiCopySamples = 256;
 
 template <int K, int COPIES>
 static void launch_hist(const MiSampledArgs& a, const MiBatch& batch, int blocks, hipStream_t s) {
@@ -375,7 +381,7 @@ void launch_mi_sampled_hist_batch(const MiSampledArgs& a, const MiBatch& batch, 
 void launch_mi_sampled_hist(const MiSampledArgs& a, int blocks, hipStream_t s) {
   const MiBatch none{};
   const size_t lds = kMiCopies * size_t(a.bins * a.bins + a.bins + 1) * sizeof(unsigned long long);
-  if (a.count / blocks >= kMiCopySamples && lds <= (size_t(64) << 10)) launch_hist<1, kMiCopies>(a, none, blocks, s);
+  if (a.count > blocks * (long long)kMiCopySamples && lds <= (size_t(64) << 10)) launch_hist<1, kMiCopies>(a, none, blocks, s);
   else launch_hist<1, 1>(a, none, blocks, s);
 }
 
