@@ -16,10 +16,10 @@ namespace fw::hip {
 //
 // The window sums of a, b, aa, bb and ab are taken in f64, every window from its own terms: the
 // product of two f32 values is exact in f64, and no sum is ever formed by subtracting a plane that
-// has left the window. So a window of zeros sums to exactly zero (which decides the degenerate
-// windows of cc.rs:270-300), a window of tiny values (the smoothed edge of a zero-padded region,
-// local variance 1e-12, where the coefficient is the largest of the image) keeps its relative
-// precision, and no scale of the image enters. The centred moments, the local CC and the
+// has left the window. So a window of zeros sums to exactly zero (and is a degenerate window of
+// cc.rs:270-300; one of another value is so within its sums' rounding, mean_of), a window of tiny
+// values (the smoothed edge of a zero-padded region, local variance 1e-12, where the coefficient is
+// the largest of the image) keeps its relative precision, and no scale of the image enters. The centred moments, the local CC and the
 // coefficients follow in f64 from one reciprocal; the derivative is the coefficient times the f32
 // central difference, rounded once to f32. Each output voxel writes both derivative directions;
 // localCC is symmetric, so one value partial serves both.
@@ -163,8 +163,9 @@ __device__ __forceinline__ double reciprocal(double v) {
   return fma(fma(-v, r, 1.0), r, r);
 }
 
-// sum / count by the count's reciprocal and one correction: exact where the quotient is (a window of
-// one value has that value as its mean, so its variance is zero, not a rounding error).
+// sum / count by the count's reciprocal and one correction: exact where the quotient is (a window of one value
+// has that value as its mean, so its centred moments are zero up to the rounding of the sums of squares, n v^2
+// 2^-53 a few times; exactly zero where those sums fit 53 bits).
 __device__ __forceinline__ double mean_of(double sum, double count, double inv_count) {
   const double q = sum * inv_count;
   return fma(fma(-q, count, sum), inv_count, q);

@@ -11,7 +11,7 @@ import pytest
 import oracle
 from fastwarp_amd._abi import Grid
 from tests import cases
-from tests.test_gpu_cc_tiles import PERMUTED
+from tests.test_gpu_cc_tiles import PERMUTED, walks
 
 pytestmark = pytest.mark.gpu
 
@@ -31,21 +31,6 @@ def pair(backend, g, f, m, radius, valid=None):
     return (v0, backend.download_field(d0)), (v1, backend.download_field(d1))
 
 
-class runs:
-    """The z runs of a tuning table (which also choose the walking kernel where there is one)."""
-
-    def __init__(self, backend, planes):
-        self.backend, self.planes = backend, planes
-
-    def __enter__(self):
-        self.backend.set_tuning("cc.tile_z", self.planes)
-        self.backend.set_tuning("cc.min_blocks", 1)
-
-    def __exit__(self, *_):
-        self.backend.set_tuning("cc.tile_z", -1)
-        self.backend.set_tuning("cc.min_blocks", -1)
-
-
 def holes(g):
     i, j, k = cases.coords(g)
     return ((i >= 3) & (j < 9) & (k != 7) & ((i + 2 * j + 3 * k) % 11 != 0)).astype(float)
@@ -63,7 +48,7 @@ def test_both_kernels_match_the_oracle(backend, axes, masked, radius):
     got = [pair(backend, g, f, m, radius, valid)]
     # a run of seven planes (shorter and longer than the windows' cycles), and one of all planes
     for planes in (7, 64):
-        with runs(backend, planes):
+        with walks(backend, planes):
             got.append(pair(backend, g, f, m, radius, valid))
     for both in got:
         for (value, field), w in zip(both, want):
@@ -93,7 +78,7 @@ def test_a_value_that_is_not_finite_stays_in_its_windows(backend, radius, bad):
         if planes is None:
             clean, got = pair(backend, g, f, m, radius), pair(backend, g, spoilt, m, radius)
         else:
-            with runs(backend, planes):
+            with walks(backend, planes):
                 clean, got = pair(backend, g, f, m, radius), pair(backend, g, spoilt, m, radius)
         for (v, d), (_, d_clean) in zip(got, clean):
             assert np.isfinite(v)
