@@ -9,8 +9,9 @@ linear-stage samples (MI). The workload is the cohort pyramid (shrink 8/4/2/1) o
 the 2 mm grid's levels, on the seeded phantom. Each candidate runs `repeats` times after a warm-up
 with every launch timed (HIP events on the context's stream), in three rounds; the knob takes the
 candidate with the least total kernel time of the op when it beats the library's default shape by
-more than MARGIN, and keeps the default (no entry) otherwise. Choices change results at most by rounding (the CC z runs
-change the order of the corrections' sums; block counts change the order of reductions).
+more than MARGIN, and keeps the default (no entry) otherwise. Choices change results at most by
+rounding (a CC z run chooses the walking kernel and the order of its windows' f64 sums; block counts
+change the order of reductions).
 """
 from __future__ import annotations
 
