@@ -1,13 +1,14 @@
 """Builds the gfx950 shared library `fastwarp_amd/lib/libfastwarp_hip.so` in-tree with hipcc.
 
 Every translation unit is compiled in parallel into `fastwarp_amd/_build/`, then linked (the CC
-kernels as one object per window radius). HIP code is compiled with the packed-FP32 instructions disabled (`-packed-fp32-ops`).
+kernels as one object per window radius and launch). HIP code is compiled with the packed-FP32 instructions disabled (`-packed-fp32-ops`).
 """
 from __future__ import annotations
 
 import os
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 HERE = Path(__file__).resolve().parent
@@ -43,12 +44,17 @@ FLAGS = [
 
 
 def _run(cmds: list[list[str]]) -> None:
-    procs = [subprocess.Popen(c, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True) for c in cmds]
+    def one(c):
+        p = subprocess.run(c, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+        return p.returncode, p.stdout
+
+    # as many at a time as there are processors (a large CC object takes about 0.5 GB)
+    with ThreadPoolExecutor(max_workers=os.cpu_count() or 1) as pool:
+        done = list(pool.map(one, cmds))
     failed = []
-    for c, p in zip(cmds, procs):
-        out, _ = p.communicate()
-        lines = [l for l in out.splitlines() if "packed-fp32-ops" not in l and "unknown target feature" not in l]
-        if p.returncode != 0:
+    for c, (code, out) in zip(cmds, done):
+        if code != 0:
+            lines = [l for l in out.splitlines() if "packed-fp32-ops" not in l and "unknown target feature" not in l]
             failed.append((c, "\n".join(lines)))
     if failed:
         for c, text in failed:
@@ -59,7 +65,8 @@ def _run(cmds: list[list[str]]) -> None:
 def objects() -> list[tuple[Path, Path, list[str]]]:
     """(source, object, further flags) of every compile step, the longest ones first."""
     cc = CSRC / "hip" / "cc.hip"
-    steps = [(cc, BUILD / f"cc_r{r}.o", [f"-DFW_CC_RADIUS={r}"]) for r in range(8, 0, -1)]
+    steps = [(cc, BUILD / f"cc_r{r}_{part}.o", [f"-DFW_CC_RADIUS={r}", f"-DFW_CC_PART={part}"])
+             for r in range(8, 0, -1) for part in (1, 0, 2)]
     return steps + [(src, BUILD / (src.name + ".o"), []) for src in SOURCES]
 
 

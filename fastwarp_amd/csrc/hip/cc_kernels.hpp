@@ -1,5 +1,5 @@
-// The fused CC kernels, templates over the window's radius. cc.hip instantiates one radius per object, so
-// that the eight compile side by side.
+// The fused CC kernels, templates over the window's radius. cc.hip instantiates one radius of one launch per
+// object, so that they compile side by side.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -434,15 +434,10 @@ static void launch_cc_one(const CcArgs& a, hipStream_t s) {
   launch((k_cc2_plane<R, M, DIAGONAL>), g, t, 0, s, a);
 }
 
-template <int R>
+template <int R, bool MASKED>
 void launch_cc_radius(const CcArgs& a, hipStream_t s) {
-  if (a.valid != nullptr) {
-    if (a.probes.diagonal) launch_cc_one<R, true, true>(a, s);
-    else launch_cc_one<R, true, false>(a, s);
-  } else {
-    if (a.probes.diagonal) launch_cc_one<R, false, true>(a, s);
-    else launch_cc_one<R, false, false>(a, s);
-  }
+  if (a.probes.diagonal) launch_cc_one<R, MASKED, true>(a, s);
+  else launch_cc_one<R, MASKED, false>(a, s);
 }
 
 template <int R, bool DIAGONAL>

@@ -23,7 +23,7 @@ LaunchEvents*& current_launch_events() {
 }
 
 // ------------------------------------------------------------------------------------------
-// CC pair: the kernels (cc_kernels.hpp) are compiled once per radius (cc.hip).
+// CC pair: the kernels (cc_kernels.hpp) are compiled once per radius and launch (cc.hip).
 // ------------------------------------------------------------------------------------------
 void launch_cc_items(const CcItems& c, hipStream_t s) {
   if (c.count < 1 || c.count > kBatchItems) return;
@@ -51,10 +51,12 @@ dim3 cc_grid(const Dims& d, int tile_z) {
 }
 
 void launch_cc_pair(const CcArgs& a, hipStream_t s) {
+  const bool masked = a.valid != nullptr;
   switch (a.radius) {
-#define FW_CC_CASE(R)          \
-  case R:                      \
-    launch_cc_radius<R>(a, s); \
+#define FW_CC_CASE(R)                             \
+  case R:                                         \
+    if (masked) launch_cc_radius<R, true>(a, s);  \
+    else launch_cc_radius<R, false>(a, s);        \
     break;
     FW_CC_CASE(1)
     FW_CC_CASE(2)

@@ -72,7 +72,7 @@ struct CcArgs {
 };
 void launch_cc_pair(const CcArgs& a, hipStream_t s);
 // The launch of one radius (1 to 8).
-template <int R>
+template <int R, bool MASKED>
 void launch_cc_radius(const CcArgs& a, hipStream_t s);
 dim3 cc_grid(const Dims& d, int tile_z);
 
