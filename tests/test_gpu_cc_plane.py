@@ -10,8 +10,11 @@ import pytest
 
 import oracle
 from fastwarp_amd._abi import Grid
+from fastwarp_amd.phantom import make_pair
+from fastwarp_amd.register import plan_2mm, register_batch, register_resident
 from tests import cases
 from tests.test_gpu_cc_tiles import PERMUTED, walks
+from tests.test_zz_no_alloc import hip, noalloc_pair
 
 pytestmark = pytest.mark.gpu
 
@@ -85,3 +88,33 @@ def test_a_value_that_is_not_finite_stays_in_its_windows(backend, radius, bad):
             assert np.array_equal(d[~near], d_clean[~near])
             if not np.isfinite(bad):
                 assert np.all(d[near] == 0.0)
+
+
+@pytest.mark.parametrize("size,radius", [((182, 218, 182), 4), ((182, 218, 90), 7), ((40, 33, 21), 8), ((96, 112, 96), 2)])
+@pytest.mark.parametrize("oblique", [0.0, 0.35])
+def test_the_pair_without_allocation_takes_the_same_launch(backend, size, radius, oblique):
+    # runs of several planes and of one, both kernels: the bits of fw_cc_pair, value included
+    g = cases.grid(size, (1.1, 0.9, 1.3), oblique=oblique)
+    f, m = cases.image(g, 7), cases.image(g, 8)
+    values, d0, d1 = noalloc_pair(hip(), g, f, m, radius)
+    (v0, e0), (v1, e1) = pair(backend, g, f, m, radius)
+    assert values[0] == v0 and values[1] == v1
+    assert np.array_equal(d0, e0) and np.array_equal(d1, e1)
+
+
+@pytest.mark.parametrize("radius,oblique", [(2, 0.35), (4, 0.35), (7, 0.35), (5, 0.0)])
+def test_batched_pairs_give_the_bits_of_single_ones(backend, radius, oblique):
+    # subjects against one template through the batched launches of both kernels (levels on both sides of the line)
+    pairs = [make_pair((96, 112, 96), 2.0, seed=30 + q) for q in range(3)]
+    g = cases.grid((96, 112, 96), (2.0, 2.0, 2.0), tuple(pairs[0].grid.origin), oblique=oblique)
+    up = lambda v: [backend.upload_image(g, v)]
+    plan = plan_2mm(1)
+    plan.set_linear([8, 5], [4, 2], [2.0, 1.0])
+    plan.set_syn([4, 3, 2], [4, 2, 1], [2.0, 1.0, 0.0])
+    plan.cc_radius = radius
+    template, moving = up(pairs[0].fixed[0]), [up(p.moving[0]) for p in pairs]
+    batch = register_batch(backend, plan, template, moving)
+    for got, mov in zip(batch, moving):
+        alone = register_resident(backend, plan, template, mov)
+        for name in ("forward", "inverse"):
+            assert np.array_equal(backend.download_field(getattr(got, name)), backend.download_field(getattr(alone, name))), name
