@@ -10,6 +10,8 @@ namespace fw::hip {
 constexpr int kCcTileX = 32, kCcTileY = 8;        // a CC block's columns and rows
 constexpr int kCcTileZ = 16, kCcMinBlocks = 512;  // where the tuning table sets only the other knob
 constexpr long long kCcCus = 256, kCcMostBlocks = 8192;
+// runs of a column, so that a batch's columns stay below the 65,536 blocks that a launch may have along z
+constexpr long long kCcMostRuns = 2048;
 
 inline long long cc_columns(int nx, int ny) {
   return (long long)((nx + kCcTileX - 1) / kCcTileX) * ((ny + kCcTileY - 1) / kCcTileY);
@@ -42,7 +44,8 @@ inline int cc_run(int nx, int ny, int nz, int radius, int max_tile, int min_bloc
   int best = nz;
   double least = 1e300;
   // at most kCcMostBlocks blocks, beyond one a tile
-  for (long long chunks = 1; chunks <= nz && (chunks == 1 || chunks * tiles <= kCcMostBlocks); ++chunks) {
+  const long long most = std::min({(long long)nz, kCcMostRuns, std::max<long long>(1, kCcMostBlocks / tiles)});
+  for (long long chunks = 1; chunks <= most; ++chunks) {
     const int t = (int)((nz + chunks - 1) / chunks);
     const long long per_cu = (tiles * ((nz + t - 1) / t) + kCcCus - 1) / kCcCus;
     const double time = double(t + 2 * radius) * cc_cu_time(per_cu, radius);
@@ -83,7 +86,7 @@ inline CcPlan cc_plan(int nx, int ny, int nz, int radius, bool masked, bool diag
   const long long tiles = cc_columns(nx, ny);
   const long long line = !diagonal ? kCcPlanes : masked ? kCcPlanesMasked : radius <= 3 ? kCcPlanesSmallRadius : kCcPlanes;
   if (walks && tiles * nz > line) return {cc_run(nx, ny, nz, radius, 0, 0), false};
-  const long long chunks = std::min<long long>(nz, std::max<long long>(1, kCcMostBlocks / tiles));
+  const long long chunks = std::min({(long long)nz, kCcMostRuns, std::max<long long>(1, kCcMostBlocks / tiles)});
   return {int((nz + chunks - 1) / chunks), true};
 }
 

@@ -1107,6 +1107,12 @@ static void cc_launches() {
         const CcPlan knob = cc_plan(24, 28, 24, radius, masked, diagonal, 5, 1);
         CHECK(knob.plane == !walks && knob.run == 5, "a table's run");
       }
+  // long thin grids: the default rules leave the pairs of a launch (8, here 16) below 65,536 blocks along z
+  for (const int nz : {2048, 2049, 4096, 100000, 1 << 20})
+    for (const bool diagonal : {false, true}) {
+      const int run = cc_plan(20, 7, nz, 4, false, diagonal, 0, 0).run;
+      CHECK(run >= 1 && 16ll * ((nz + run - 1) / run) < 65536, "blocks along z");
+    }
   CHECK(cc_plan(96, 112, 96, 4, false, true, 0, 0).plane && !cc_plan(96, 112, 97, 5, true, true, 0, 0).plane, "the lines");
   ok("cc_launches");
 }
